@@ -263,6 +263,10 @@ __device__ void fused_path(const FusedIn& in, const FusedOut& out, FusedCtl* ctl
     const int64_t vb = in.verb_off[p], ve = in.verb_off[p + 1];
     const int64_t pb = in.point_off[p], pe = in.point_off[p + 1];
     const int64_t wb = in.weight_off[p], we = in.weight_off[p + 1];
+    if (ADJ && (ve - vb > A_VCAP || pe - pb > A_PCAP)) {  // over one wave's limits whatever its lines are
+        if (lane == 0) deferred[atomicAdd(&ctl->deferred, 1u)] = (uint32_t)p;  // (the adjoint's large path)
+        return;
+    }
     int32_t aox = 0, aoy = 0;
     const Xform X = ADJ ? adjoint_local_xform(in, p, &aox, &aoy) : in.xf[p];
 
@@ -378,8 +382,7 @@ __device__ void fused_path(const FusedIn& in, const FusedOut& out, FusedCtl* ctl
     if (has_lines && !full && bminx <= bmaxx)
         grid_from_box(true, false, (int32_t)floorf(bminx), (int32_t)floorf(bminy), (int32_t)floorf(bmaxx),
                       (int32_t)floorf(bmaxy), &tx0, &ty0, &GW, &GH);
-    if (overflow || full || GW > F_GRID || GH > F_GRID ||
-        (ADJ && (ve - vb > A_VCAP || pe - pb > A_PCAP))) {
+    if (overflow || full || GW > F_GRID || GH > F_GRID) {
         if (lane == 0) deferred[atomicAdd(&ctl->deferred, 1u)] = (uint32_t)p;  // (the adjoint's large path)
         return;
     }
@@ -1083,19 +1086,29 @@ int run_batched(Context* ctx, const SegInput& in, OutputDesc& out, hipStream_t s
     return st;
 }
 
-// The large-path adjoint of path p (one path over the whole device; see
-// adjoint_large.inc).  `hp`: 2 KiB of pinned host memory for the read-backs.
-static int run_adjoint_large(const FusedIn& fi, const AdjArgs& a, int64_t p, hipStream_t s, BatchedState* B,
-                             uint8_t* hp) {
-    int64_t* off = reinterpret_cast<int64_t*>(hp);
-    HIPCHK_RET(hipMemcpyAsync(off, fi.verb_off + p, 16, hipMemcpyDeviceToHost, s));
-    HIPCHK_RET(hipMemcpyAsync(off + 2, fi.point_off + p, 16, hipMemcpyDeviceToHost, s));
-    HIPCHK_RET(hipStreamSynchronize(s));
-    const int64_t nv = off[1] - off[0], np = off[3] - off[2];
+// The large-path adjoint of path p, of nv commands and np points (one path over
+// the whole device; see adjoint_large.inc).  `hp`: 2 KiB of pinned host memory
+// for the read-back.  The call's error word (in the control block at the start
+// of large_cmd, whose room for every path of the call the caller has ensured)
+// keeps what the last passes of a path report; the caller reads it once.
+constexpr size_t AL_CTL_BYTES = 256;  // box[4], nt, err, acc[8]
+static size_t al_command_bytes(int64_t nv, int64_t np) {
+    return AL_CTL_BYTES + 3 * ((size_t)nv * 8 + 256) + ((size_t)(nv + 1) * 4 + 256) + 2 * ((size_t)np * 4 + 256) +
+           ((size_t)nv * 48 + 256);
+}
+static int al_status(uint32_t err) {
+    if (err & ERR_INPUT) return -1;
+    if (err & ERR_FLATTEN) return -5;
+    if (err & ERR_CAPACITY) return -7;  // coordinates beyond the 16-bit pixel range
+    if (err & ERR_BBOX) return -3;
+    return 0;
+}
+static int run_adjoint_large(const FusedIn& fi, const AdjArgs& a, int64_t p, int64_t nv, int64_t np, hipStream_t s,
+                             BatchedState* B, uint8_t* hp) {
     if (nv < 0 || np < 0) return -1;
-    // command scratch: cg, cmv, cw | cl | pcmd | slot | box, err, nt | acc
+    // command scratch: box, nt, err, acc | cg, cmv, cw | cl | pcmd | closer | slot
     auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
-    size_t o = 0;
+    size_t o = AL_CTL_BYTES;
     const size_t o_cg = o;
     o = al(o + (size_t)nv * 8);
     const size_t o_cmv = o;
@@ -1106,13 +1119,10 @@ static int run_adjoint_large(const FusedIn& fi, const AdjArgs& a, int64_t p, hip
     o = al(o + (size_t)(nv + 1) * 4);
     const size_t o_pcmd = o;
     o = al(o + (size_t)np * 4);
+    const size_t o_closer = o;
+    o = al(o + (size_t)np * 4);
     const size_t o_slot = o;
     o = al(o + (size_t)nv * 48);
-    const size_t o_ctl = o;  // box[4], err, nt
-    o = al(o + 32);
-    const size_t o_acc = o;
-    o = al(o + 8 * 8);
-    HIPCHK_RET(B->large_cmd.ensure(o));
     uint8_t* c = B->large_cmd.as<uint8_t>();
     LargeAdj A;
     memset(&A, 0, sizeof(A));
@@ -1121,28 +1131,28 @@ static int run_adjoint_large(const FusedIn& fi, const AdjArgs& a, int64_t p, hip
     A.cw = reinterpret_cast<int64_t*>(c + o_cw);
     A.cl = reinterpret_cast<uint32_t*>(c + o_cl);
     A.pcmd = reinterpret_cast<uint32_t*>(c + o_pcmd);
+    A.closer = reinterpret_cast<uint32_t*>(c + o_closer);
     A.slot = reinterpret_cast<float*>(c + o_slot);
-    A.box = reinterpret_cast<unsigned*>(c + o_ctl);
-    A.err = reinterpret_cast<uint32_t*>(c + o_ctl + 16);
-    A.nt = reinterpret_cast<uint32_t*>(c + o_ctl + 20);
-    A.acc = reinterpret_cast<double*>(c + o_acc);
+    A.box = reinterpret_cast<unsigned*>(c);
+    A.nt = reinterpret_cast<uint32_t*>(c + 16);
+    A.err = reinterpret_cast<uint32_t*>(c + 20);
+    A.acc = reinterpret_cast<double*>(c + 64);
     HIPCHK_RET(hipMemsetAsync(A.box, 0xff, 8, s));        // min x, min y
-    HIPCHK_RET(hipMemsetAsync(A.box + 2, 0, 16, s));      // max x, max y, err, nt
+    HIPCHK_RET(hipMemsetAsync(A.box + 2, 0, 12, s));      // max x, max y, nt
     HIPCHK_RET(hipMemsetAsync(A.acc, 0, 8 * 8, s));
+    // a wave per workgroup where a thread's work is long and threads are few (a
+    // command, a line): 1,400 commands or 30,000 lines then reach every CU
     const int T = 256;
-    const unsigned gv = (unsigned)std::max<int64_t>(1, (nv + T - 1) / T);
+    const unsigned gv = (unsigned)std::max<int64_t>(1, (nv + WAVE - 1) / WAVE);
     hipLaunchKernelGGL(k_al_cmds, dim3(1), dim3(1024), 0, s, fi, p, A);
-    hipLaunchKernelGGL(k_al_count, dim3(gv), dim3(T), 0, s, fi, p, A);
+    hipLaunchKernelGGL(k_al_count, dim3(gv), dim3(WAVE), 0, s, fi, p, A);
     hipLaunchKernelGGL(k_al_scan, dim3(1), dim3(1024), 0, s, fi, p, A);
     HIPCHK_RET(hipGetLastError());
     uint32_t* hc = reinterpret_cast<uint32_t*>(hp + 64);
     HIPCHK_RET(hipMemcpyAsync(hc, A.cl + nv, 4, hipMemcpyDeviceToHost, s));
-    HIPCHK_RET(hipMemcpyAsync(hc + 1, A.box, 24, hipMemcpyDeviceToHost, s));  // box[4], err, nt
+    HIPCHK_RET(hipMemcpyAsync(hc + 1, A.box, 24, hipMemcpyDeviceToHost, s));  // box[4], nt, err
     HIPCHK_RET(hipStreamSynchronize(s));
-    const uint32_t e1 = hc[5];
-    if (e1 & ERR_INPUT) return -1;
-    if (e1 & ERR_FLATTEN) return -5;
-    if (e1 & ERR_CAPACITY) return -7;  // coordinates beyond the 16-bit pixel range
+    if (const int st = al_status(hc[6])) return st;
     const int64_t L = hc[0];
     if (L >= AL_MAX_LINES) return -7;
     int32_t tx0 = 0, ty0 = 0, GW = 0, GH = 0;
@@ -1192,25 +1202,19 @@ static int run_adjoint_large(const FusedIn& fi, const AdjArgs& a, int64_t p, hip
     A.GH = GH;
     A.ow = ow;
     if (o_g > o_occ) HIPCHK_RET(hipMemsetAsync(gbuf + o_occ, 0, o_g - o_occ, s));  // occ, sums, crossings, spans
-    const unsigned gl = (unsigned)std::max<int64_t>(1, (L + T - 1) / T);
-    const unsigned gp = (unsigned)std::max<int64_t>(1, (np + T - 1) / T);
-    const unsigned gr = (unsigned)std::max<int64_t>(1, ((int64_t)GH * TILE + T - 1) / T);
-    hipLaunchKernelGGL(k_al_lines, dim3(gv), dim3(T), 0, s, fi, p, A);
-    if (L > 0) hipLaunchKernelGGL(k_al_fwd, dim3(gl), dim3(T), 0, s, L, A);
+    const unsigned gl = (unsigned)std::max<int64_t>(1, (L + WAVE - 1) / WAVE);
+    const unsigned gp = (unsigned)std::max<int64_t>(1, (np + AL_GT - 1) / AL_GT);
+    hipLaunchKernelGGL(k_al_lines, dim3(gv), dim3(WAVE), 0, s, fi, p, A);
+    if (L > 0) hipLaunchKernelGGL(k_al_fwd, dim3(gl), dim3(WAVE), 0, s, L, A);
     hipLaunchKernelGGL(k_al_spans, dim3(1), dim3(1024), 0, s, A);
-    if (GH > 0) hipLaunchKernelGGL(k_al_rows, dim3(gr), dim3(T), 0, s, fi, A, a, p);
+    if (GH > 0) hipLaunchKernelGGL(k_al_rows, dim3(GH), dim3(512), 0, s, fi, A, a, p);
     // target tiles: one thread each (their count is the caller's, bounded by its capacity)
     hipLaunchKernelGGL(k_al_target, dim3(4096), dim3(T), 0, s, fi, A, a, p);
-    if (L > 0) hipLaunchKernelGGL(k_al_bwd, dim3(gl), dim3(T), 0, s, L, A);
-    hipLaunchKernelGGL(k_al_cmd_bwd, dim3(gv), dim3(T), 0, s, fi, p, A);
-    if (np > 0) hipLaunchKernelGGL(k_al_gather, dim3(gp), dim3(T), 0, s, fi, p, A, a);
+    if (L > 0) hipLaunchKernelGGL(k_al_bwd, dim3(gl), dim3(WAVE), 0, s, L, A);
+    hipLaunchKernelGGL(k_al_cmd_bwd, dim3(gv), dim3(WAVE), 0, s, fi, p, A);
+    if (np > 0) hipLaunchKernelGGL(k_al_gather, dim3(gp), dim3(AL_GT), 0, s, fi, p, A, a);
     hipLaunchKernelGGL(k_al_final, dim3(1), dim3(1), 0, s, A, a, p);
     HIPCHK_RET(hipGetLastError());
-    HIPCHK_RET(hipMemcpyAsync(hc, A.err, 4, hipMemcpyDeviceToHost, s));
-    HIPCHK_RET(hipStreamSynchronize(s));
-    if (hc[0] & ERR_INPUT) return -1;
-    if (hc[0] & ERR_FLATTEN) return -5;
-    if (hc[0] & ERR_BBOX) return -3;
     return 0;
 }
 
@@ -1286,14 +1290,27 @@ int run_adjoint(Context* ctx, const SegInput& in, const AdjTarget& tgt, float* l
     // the paths over one wave's limits, one at a time over the whole device
     const uint32_t n_large = hc->deferred;
     if (n_large) {
-        std::vector<uint32_t> ids(n_large);
-        HIPCHK_RET(hipMemcpy(ids.data(), large, (size_t)n_large * 4, hipMemcpyDeviceToHost));
-        std::sort(ids.begin(), ids.end());
+        HIPCHK_RET(B->large_grid.ensure((size_t)n_large * sizeof(AlSize)));
+        AlSize* dsz = B->large_grid.as<AlSize>();
+        hipLaunchKernelGGL(k_al_sizes, dim3((n_large + 255) / 256), dim3(256), 0, s, fi, large, n_large, dsz);
+        HIPCHK_RET(hipGetLastError());
+        std::vector<AlSize> sz(n_large);
+        HIPCHK_RET(hipMemcpyAsync(sz.data(), dsz, (size_t)n_large * sizeof(AlSize), hipMemcpyDeviceToHost, s));
+        HIPCHK_RET(hipStreamSynchronize(s));
+        std::sort(sz.begin(), sz.end(), [](const AlSize& x, const AlSize& y) { return x.path < y.path; });
+        size_t room = 0;
+        for (const AlSize& z : sz) room = std::max(room, al_command_bytes(std::max<int64_t>(z.nv, 0), std::max<int64_t>(z.np, 0)));
+        HIPCHK_RET(B->large_cmd.ensure(room));
+        HIPCHK_RET(hipMemsetAsync(B->large_cmd.p, 0, AL_CTL_BYTES, s));
         uint8_t* hp = reinterpret_cast<uint8_t*>(ctx->host_pinned) + 2048;
-        for (uint32_t id : ids) {
-            const int st = run_adjoint_large(fi, a, (int64_t)id, s, B, hp);
+        for (const AlSize& z : sz) {
+            const int st = run_adjoint_large(fi, a, z.path, z.nv, z.np, s, B, hp);
             if (st) return st;
         }
+        uint32_t* he = reinterpret_cast<uint32_t*>(hp);
+        HIPCHK_RET(hipMemcpyAsync(he, B->large_cmd.as<uint8_t>() + 20, 4, hipMemcpyDeviceToHost, s));
+        HIPCHK_RET(hipStreamSynchronize(s));
+        return al_status(*he);
     }
     return 0;
 }
