@@ -862,24 +862,34 @@ __global__ __launch_bounds__(WAVE) void k_tile_counts(TileArgs a) {
 
 // Emit pass of the tile stage: one wave per tile row, walking the row's
 // groups (bins, rasterizer.rs:213-265) in key order.  The row's sort entries
-// are taken TR_BLOCK at a time and each of the first TR_BLOCK lanes replays
-// one run into LDS: its increments in step order, and a 64-byte map from
-// pixel to step (a run stays inside one 8x8 tile and the DDA never revisits a
-// pixel, so a run has at most 15 increments, at distinct pixels).  Lane p then
-// owns pixel p of the tile: for each run in sorted order it looks its pixel up
-// in the run's map and adds the increment found there to its register sums,
-// so every pixel's f32 sums follow the sorted order exactly
-// (rasterizer.rs:221-228), with no read-modify-write through LDS.  At the end
-// of a tile the row carry is folded across the 8 lanes of each pixel row in x
-// order, the alphas quantised and stored (rasterizer.rs:230-250), and a span
+// are taken TR_BLOCK at a time and each lane replays one run into LDS: its
+// increments in step order, its first pixel, and its bit in the `hit` words of
+// the pixels it visits.  A run stays inside one 8x8 tile and its walk moves one
+// pixel along one axis per step, so it has at most 15 increments, at distinct
+// pixels, and the increment at a pixel is the one whose step is the pixel's
+// distance |dx| + |dy| from the run's first pixel: no map from pixel to step is
+// needed.  Each lane then owns a pixel of the tile and adds, for the set bits of
+// its hit words among the tile's runs, in sorted order, the increments found
+// there to its register sums, so every pixel's f32 sums follow the sorted order
+// exactly (rasterizer.rs:221-228), with no read-modify-write through LDS.  At
+// the end of a tile the row carry is folded across the 8 lanes of each pixel row
+// in x order, the alphas quantised and stored (rasterizer.rs:230-250), and a span
 // is written where the previous tile of the row is more than one tile to the
 // left and the winding after it is non-zero (rasterizer.rs:252-264).
-constexpr int TR_SLOTS = 16;  // increments per run slot
-constexpr int TR_BLOCK = 32;  // runs replayed per block (6 KB of LDS per wave; 16 and 64 measured slower)
-// (Padding these rows against the lane-strided bank conflicts of the replay
-// was measured slower: the replay is a small part of the kernel.)
-constexpr int TR_SSTR = TR_SLOTS;  // float2 per run slot row
-constexpr int TR_MSTR = 64;        // bytes per run map row
+//
+// Bound: VALU issue of the replays and, for a row alone on its SIMD, the chain of
+// dependent loads (entry, record, line) and steps.  So: 64 runs replayed at once
+// (a wave's worth; 32 left half the lanes idle), 8.2 KB of LDS per wave instead
+// of 6 KB for 32 runs (no 64-byte pixel map to clear, fill and search per run), a
+// pixel visits only the runs that hit it (the most hits of a tile's pixels, about
+// 4, instead of its runs, about 11), the next block's records and lines load
+// while this one is added, and the carry moves by DPP instead of eight LDS
+// permutes.
+// Measured against the 32-run kernel with maps: 120 -> 45 us on a line of 61
+// glyphs, 422 -> 220 us on 10,000 glyphs, 2,684 -> 1,000 us on 24 star blobs of
+// 1,000-20,000 cubics.
+constexpr int TR_SLOTS = 15;  // increments per run
+constexpr int TR_BLOCK = WAVE;  // runs replayed per block
 
 __device__ inline uint32_t rl(uint32_t v, int j) { return (uint32_t)__builtin_amdgcn_readlane((int)v, j); }
 
@@ -902,10 +912,62 @@ static inline uint32_t row_grid(int64_t rows, int64_t cap) {
     return (uint32_t)g;
 }
 
+// The increments of a run from the DDA state at its first one (p0: that
+// increment's start point) into `inc` in step order, and the run's bit into the
+// hit words of its pixels; CARRY: every active lane's line is finite, so each
+// increment's start point is the previous one's end point (see
+// dda_increment_carried).
+template <bool CARRY>
+__device__ inline void tr_replay_steps(float2* inc, uint32_t* hit, uint32_t bit, Dda& d, V2 p0, bool finite,
+                                       Counters* cnt) {
+    uint32_t lx = (uint32_t)(d.x & 7), ly = (uint32_t)(d.y & 7);
+    const uint32_t lxd = (uint32_t)(int32_t)d.x_dir, lyd = (uint32_t)(int32_t)d.y_dir;
+    bool ended = false;
+    for (int k = 0; k < TR_SLOTS; k++) {
+        float area, height;
+        dda_increment_carried(d, p0, CARRY || finite, area, height);
+        inc[k] = make_float2(area, height);
+        atomicOr(&hit[(ly << 3) | lx], bit);
+        // dda_step, with the in-tile pixel moved alongside
+        float c;
+        if (d.row_t1 < d.col_t1) {
+            c = d.row_t1;
+            d.row_t1 = fminf(d.row_t1 + d.y_step, 1.0f);
+            d.y = wrap16(d.y + d.y_dir);
+            ly += lyd;
+        } else {
+            c = d.col_t1;
+            d.col_t1 = fminf(d.col_t1 + d.x_step, 1.0f);
+            d.x = wrap16(d.x + d.x_dir);
+            lx += lxd;
+        }
+        d.t0 = c;
+        if (c == 1.0f || (lx | ly) > 7u) {
+            ended = true;
+            break;
+        }
+    }
+    if (!ended) atomicOr(&cnt->error, (uint32_t)ERR_REPLAY);
+}
+
+// The lane's value of v from DPP_CTRL's source lane; `old` where there is none.
+template <int DPP_CTRL>
+__device__ inline float dpp_f(float old, float v) {
+    return __int_as_float(
+        __builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(v), DPP_CTRL, 0xf, 0xf, false));
+}
+constexpr int DPP_ROW_SHR2 = 0x112, DPP_ROW_ROR2 = 0x122;  // within each 16 lanes
+
 __global__ __launch_bounds__(WAVE) void k_tile_rows(TileArgs a) {
-    __shared__ float2 inc[TR_BLOCK * TR_SSTR];
-    __shared__ __align__(16) uint8_t smap[TR_BLOCK * TR_MSTR];  // run j, pixel p -> step + 1 (0: not visited)
+    __shared__ float2 inc[TR_BLOCK * TR_SLOTS];
+    __shared__ uint32_t hit[2][64];        // pixel p, bit j: run 32 w + j visits p
+    __shared__ uint16_t first[TR_BLOCK];   // a run's first pixel, x | y << 8
     const int lane = threadIdx.x;
+    // Lane -> pixel: 16 lanes hold two pixel rows interleaved, so that a move of
+    // two lanes is the next pixel of the same row and the first two lanes, which
+    // have no source, keep the carry.
+    const uint32_t px = (uint32_t)(lane >> 1) & 7u, py = (uint32_t)((lane >> 4) << 1) | (uint32_t)(lane & 1);
+    const uint32_t pix = (py << 3) | px, pos = px | (py << 8);
     const uint32_t xmask = (1u << a.xbits) - 1;
     for (int64_t row = xcd_first_row(); row < a.n_rows; row += gridDim.x) {
         const PathGrid G = a.grid[a.row_path[row]];
@@ -917,7 +979,7 @@ __global__ __launch_bounds__(WAVE) void k_tile_rows(TileArgs a) {
         const uint32_t row_tiles = (uint32_t)(off >> 32), row_spans = (uint32_t)off;
         const uint32_t E_hi = a.gbegin[ge];
         int32_t winding = a.row_wb[row];
-        float carry = 0.0f;  // of the lane's pixel row
+        float carry = 0.0f;  // of the lane's pixel row, in its first lane
         uint32_t nt = 0, ns = 0;
         bool have_prev = false;
         int32_t prev_tx = 0, prev_w = 0;
@@ -935,8 +997,22 @@ __global__ __launch_bounds__(WAVE) void k_tile_rows(TileArgs a) {
         };
         load_groups();
         uint32_t e = a.gbegin[gb];
-        uint32_t ebase = e + TR_BLOCK;  // no entry block loaded yet
-        float pa = 0.0f, ph = 0.0f;     // this lane's pixel sums for the current tile
+        // the block after the current one: its entries' values, records and lines
+        auto load_val = [&](uint32_t base) {
+            const uint32_t ei = base + (uint32_t)lane;
+            return ei < E_hi ? a.vals[ei] : 0x80000000u;
+        };
+        auto load_rec = [&](uint32_t v) { return v >> 31 ? RunRec{0, 0, 0.0f, 0.0f} : a.recs[v]; };
+        auto load_line = [&](uint32_t v, const RunRec& r) {
+            return v >> 31 ? make_float4(0, 0, 0, 0) : a.lines[r.line & 0x7fffffffu];
+        };
+        uint32_t nv = load_val(e);
+        RunRec nr = load_rec(nv);
+        float4 nl = load_line(nv, nr);
+        uint32_t nv2 = load_val(e + TR_BLOCK);
+        uint32_t next = e, ebase = 0;     // first entry of the next and of the current block
+        uint32_t h0 = 0, h1 = 0;          // this pixel's hit words of the current block
+        float pa = 0.0f, ph = 0.0f;       // this pixel's sums of the current tile
         for (uint32_t g = gb; g < ge; g++) {
             if (g - gbase >= (uint32_t)WAVE) {
                 gbase = g;
@@ -945,7 +1021,7 @@ __global__ __launch_bounds__(WAVE) void k_tile_rows(TileArgs a) {
             const int j = (int)(g - gbase);
             const uint32_t key = rl(gk, j), hr = rl(ghr, j), g_end = rl(gend, j);
             winding += (int32_t)rl((uint32_t)gsg, j);
-            if (!hr) {  // tile-row crossings only
+            if (!hr) {  // tile-row crossings only (a block's entries are taken in order all the same)
                 e = g_end;
                 continue;
             }
@@ -960,83 +1036,80 @@ __global__ __launch_bounds__(WAVE) void k_tile_rows(TileArgs a) {
                 ns++;
             }
             while (e < g_end) {
-                if (e - ebase >= (uint32_t)TR_BLOCK) {
+                while (e >= next) {
                     // (c) replay the next TR_BLOCK entries, one run per lane
-                    ebase = e;
-                    __syncthreads();  // the previous block's maps are read
-                    if (lane < TR_BLOCK) {
-                        uint4* row_map = reinterpret_cast<uint4*>(smap + lane * TR_MSTR);
-#pragma unroll
-                        for (int k = 0; k < TR_MSTR / 16; k++) row_map[k] = make_uint4(0, 0, 0, 0);
-                        const uint32_t ei = ebase + (uint32_t)lane;
-                        const uint32_t v = ei < E_hi ? a.vals[ei] : 0x80000000u;
-                        if (!(v >> 31)) {
-                            const RunRec r = a.recs[v];
-                            const float4 L = a.lines[r.line & 0x7fffffffu];
-                            Dda d;
-                            const V2 last = mk(L.x, L.y), point = mk(L.z, L.w);
-                            if (r.line >> 31) {
-                                dda_init(d, last, point);
-                            } else {
-                                dda_consts(d, last, point);
-                                d.x = (int16_t)(r.xy & 0xffffu);
-                                d.y = (int16_t)(r.xy >> 16);
-                                d.row_t1 = r.row_t1;
-                                d.col_t1 = r.col_t1;
-                                d.t0 = 0.0f;
-                                dda_step(d);
-                            }
-                            const int16_t rtx = div8(d.x), rty = div8(d.y);
-                            const bool finite = line_finite(last, point);
-                            V2 p0 = dda_point(d, d.t0);
-                            bool ended = false;
-                            for (int k = 0; k < TR_SLOTS; k++) {
-                                float area, height;
-                                dda_increment_carried(d, p0, finite, area, height);
-                                inc[lane * TR_SSTR + k] = make_float2(area, height);
-                                smap[lane * TR_MSTR + (((d.y & 7) << 3) | (d.x & 7))] = (uint8_t)(k + 1);
-                                if (dda_step(d) || div8(d.x) != rtx || div8(d.y) != rty) {
-                                    ended = true;
-                                    break;
-                                }
-                            }
-                            if (!ended) atomicOr(&a.cnt->error, (uint32_t)ERR_REPLAY);
-                        }
-                    }
+                    ebase = next;
+                    next += TR_BLOCK;
+                    const uint32_t v = nv;
+                    const RunRec r = nr;
+                    const float4 L = nl;
+                    nv = nv2;
+                    nr = load_rec(nv);
+                    __syncthreads();  // the previous block's increments are read
+                    hit[0][lane] = 0;
+                    hit[1][lane] = 0;
                     __syncthreads();
+                    if (!(v >> 31)) {
+                        Dda d;
+                        const V2 last = mk(L.x, L.y), point = mk(L.z, L.w);
+                        if (r.line >> 31) {
+                            dda_init(d, last, point);
+                        } else {
+                            dda_consts(d, last, point);
+                            d.x = (int16_t)(r.xy & 0xffffu);
+                            d.y = (int16_t)(r.xy >> 16);
+                            d.row_t1 = r.row_t1;
+                            d.col_t1 = r.col_t1;
+                            d.t0 = 0.0f;
+                            dda_step(d);
+                        }
+                        const bool finite = line_finite(last, point);
+                        const V2 p0 = dda_point(d, d.t0);
+                        first[lane] = (uint16_t)((d.x & 7) | ((d.y & 7) << 8));
+                        float2* out = inc + lane * TR_SLOTS;
+                        uint32_t* hw = hit[lane >> 5];
+                        const uint32_t bit = 1u << (lane & 31);
+                        if (__ballot(!finite) == 0) tr_replay_steps<true>(out, hw, bit, d, p0, finite, a.cnt);
+                        else tr_replay_steps<false>(out, hw, bit, d, p0, finite, a.cnt);
+                    }
+                    nl = load_line(nv, nr);
+                    nv2 = load_val(next + TR_BLOCK);
+                    __syncthreads();
+                    h0 = hit[0][pix];
+                    h1 = hit[1][pix];
                 }
-                // up to 8 runs of this block at a time, added in sorted order
-                const uint32_t jr = e - ebase;
-                const uint32_t m = min(min(8u, g_end - e), (uint32_t)TR_BLOCK - jr);
-                uint32_t k8[8];
-#pragma unroll
-                for (int i = 0; i < 8; i++) k8[i] = (uint32_t)i < m ? smap[(jr + i) * TR_MSTR + lane] : 0u;
-#pragma unroll
-                for (int i = 0; i < 8; i++) {
-                    if (k8[i]) {
-                        const float2 v = inc[(jr + i) * TR_SSTR + k8[i] - 1];
+                // the tile's runs of this block, added in sorted order
+                const uint32_t j0 = e - ebase, j1 = min(g_end, next) - ebase;
+                auto add_runs = [&](uint32_t h, uint32_t lo, uint32_t hi, const uint16_t* fst, const float2* incs) {
+                    uint32_t m = h & (0xffffffffu << lo) & (0xffffffffu >> (32u - hi));
+                    while (m) {
+                        const uint32_t r = (uint32_t)__ffs((int)m) - 1u;
+                        m &= m - 1u;
+                        // |dx| + |dy| from the run's first pixel, by bytes
+                        const float2 v = incs[__builtin_amdgcn_sad_u8((uint32_t)fst[r], pos, r * (uint32_t)TR_SLOTS)];
                         pa = pa + v.x;
                         ph = ph + v.y;
                     }
-                }
-                e += m;
+                };
+                if (j0 < 32u) add_runs(h0, j0, min(j1, 32u), first, inc);
+                if (j1 > 32u) add_runs(h1, j0 > 32u ? j0 - 32u : 0u, j1 - 32u, first + 32, inc + 32 * TR_SLOTS);
+                e = ebase + j1;
             }
-            // (d)(e) lane = pixel (y = lane >> 3, x = lane & 7)
-            const int x = lane & 7;
-            float fold = carry, mine = 0.0f;
+            // (d)(e) the fold along each pixel row: after k moves the lanes of
+            // pixels 0..k hold ((carry + h0) + h1) ..., the later ones not yet
+            float mine = carry, t = carry + ph;
 #pragma unroll
-            for (int k = 0; k < 8; k++) {
-                const float hk = __shfl(ph, (lane & ~7) | k, WAVE);
-                if (x == k) mine = fold;
-                fold = fold + hk;
+            for (int k = 1; k < TILE; k++) {
+                mine = dpp_f<DPP_ROW_SHR2>(carry, t);
+                t = mine + ph;
             }
-            carry = fold;
-            const float q = fminf(fabsf(mine + pa) * 256.0f, 255.0f);
-            if (a.tile_cov) a.tile_cov[(size_t)(row_tiles + nt) * 64 + lane] = fminf(fabsf(mine + pa), 1.0f);
+            carry = dpp_f<DPP_ROW_ROR2>(t, t);
+            const float cov = fabsf(mine + pa);
+            const uint32_t ti = row_tiles + nt;
+            if (a.tile_cov) a.tile_cov[(size_t)ti * 64 + pix] = fminf(cov, 1.0f);
+            a.tile_alpha[(size_t)ti * 64 + pix] = (uint8_t)(uint32_t)fminf(cov * 256.0f, 255.0f);
             pa = 0.0f;
             ph = 0.0f;
-            const uint32_t ti = row_tiles + nt;
-            a.tile_alpha[(size_t)ti * 64 + lane] = (uint8_t)(uint32_t)q;
             if (lane == 0) {
                 a.tile_xy[2 * ti] = (int16_t)(tx * TILE);
                 a.tile_xy[2 * ti + 1] = (int16_t)(ty * TILE);
