@@ -126,8 +126,7 @@ struct Context {
     DBuf counters, totals;
     DBuf call_error;  // emit-phase error bits of the current plain call (all passes)
     DBuf keys[2], vals[2], records, rs_counts;
-    DBuf grp_begin, grp_key, grp_hasrun, grp_sign;
-    DBuf row_gbegin, row_gend, row_sign, row_wb, row_path, row_cnt, row_off;
+    DBuf row_begin, row_end, row_sign, row_wb, row_path, row_cnt, row_off;
     DBuf split_off;  // rebased per-path offsets of a path range (run_plain's split)
     DBuf u_pwbase, u_rwbase, u_bcnt, u_bbeg, u_bcur;  // unordered tile stage: window buckets
     double split_ratio = 2.0;  // how far the last pass that had to split was over its limits

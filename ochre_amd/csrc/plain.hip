@@ -461,9 +461,10 @@ struct StoreRowBase {
     __device__ void operator()(int64_t i, uint32_t excl, uint32_t) const { g[i].row_base = excl; }
 };
 
-// In the unordered tile stage the run that starts a line has no record (its
-// replay starts where the line does): its entry's value is the line; the
-// value of a later run is its record's index with RT_REC set.  (Replaying
+// A sort entry's value: bit 31 a tile-row crossing (its sign in the low byte).
+// Else a run: the one that starts a line has no record (its replay starts where
+// the line does), its value is the line; a later run's is its record's index
+// with RT_REC set.  (Replaying
 // every run from its line's start instead of keeping records measured slower:
 // the extra steps cost more than the records' writes and gathers.)
 constexpr uint32_t RT_REC = 0x40000000u;
@@ -512,7 +513,6 @@ struct CountSink {
 struct EmitSink {
     uint32_t line;
     uint32_t entry, run_idx;
-    bool unordered;     // the unordered tile stage's entries (see RT_FIRST_RUN)
     PathGrid g;
     uint32_t xbits;
     uint32_t* keys;
@@ -533,14 +533,14 @@ struct EmitSink {
         uint32_t k = 0;
         key_of(tx, ty, &k);
         keys[entry] = k;
-        if (unordered && start) {
+        if (start) {
             vals[entry] = line;
             entry++;
             return;
         }
-        vals[entry] = run_idx | (unordered ? RT_REC : 0u);
+        vals[entry] = run_idx | RT_REC;
         RunRec r;
-        r.line = line | (start ? 0x80000000u : 0u);
+        r.line = line;
         r.xy = (uint32_t)(uint16_t)d.x | ((uint32_t)(uint16_t)d.y << 16);
         r.row_t1 = d.row_t1;
         r.col_t1 = d.col_t1;
@@ -562,7 +562,7 @@ struct DdaArgs {
     const float4* lines;
     const uint32_t* line_path;
     int64_t n_lines;
-    uint64_t* line_cnt;        // count pass: (runs << 32) | entries per line, read by the emit pass
+    uint64_t* line_cnt;        // count pass: (records << 32) | entries per line, read by the emit pass
     const PathGrid* grid;
     uint32_t xbits;
     uint32_t* keys;
@@ -570,8 +570,7 @@ struct DdaArgs {
     RunRec* recs;
     Counters* cnt;
     uint64_t* blk_entries;     // count pass: the entries of each block's lines
-    uint64_t* blk_cnt;         // count pass: each block's (runs << 32) | entries; emit pass: exclusive offsets
-    bool unordered;            // the unordered tile stage's entries (RT_REC)
+    uint64_t* blk_cnt;         // count pass: each block's (records << 32) | entries; emit pass: exclusive offsets
 };
 
 
@@ -592,8 +591,8 @@ __global__ __launch_bounds__(256) void k_dda(DdaArgs a) {
             s.cnt = a.cnt;
             if (!line_counts(mk(L.x, L.y), mk(L.z, L.w), s.runs, s.entries))
                 walk_line(mk(L.x, L.y), mk(L.z, L.w), s);
-            const uint32_t runs = (a.unordered && s.runs) ? s.runs - 1u : s.runs;  // no record for the first run
-            c = ((uint64_t)runs << 32) | s.entries;
+            const uint32_t recs = s.runs ? s.runs - 1u : 0u;  // no record for the first run
+            c = ((uint64_t)recs << 32) | s.entries;
             a.line_cnt[l] = c;
             e = s.entries;
         }
@@ -633,7 +632,6 @@ __global__ __launch_bounds__(256) void k_dda(DdaArgs a) {
         s.vals = a.vals;
         s.recs = a.recs;
         s.cnt = a.cnt;
-        s.unordered = a.unordered;
         if (!walk_line_tiles(mk(L.x, L.y), mk(L.z, L.w), s)) walk_line(mk(L.x, L.y), mk(L.z, L.w), s);
     }
 }
@@ -659,81 +657,76 @@ struct StoreU64 {
     __device__ void operator()(int64_t i, uint64_t excl, uint64_t) const { p[i] = excl; }
 };
 
-// ------------------------------------------------ groups and tile rows
+// ------------------------------------------------ tile rows
 
-struct LoadGroupStart {
-    const uint32_t* keys;
-    __device__ uint32_t operator()(int64_t i) const { return (i == 0 || keys[i] != keys[i - 1]) ? 1u : 0u; }
-};
-// Group tables from the sorted entries: each group's first entry and key,
-// whether it holds a run, and its crossing sum.  A thread's chunk of
-// consecutive entries is taken at once: one sign atomic and one run flag per
-// group the chunk touches, instead of one per entry.
-struct StoreGroup {
-    using chunk_tag = void;
-    const uint32_t* keys;
-    const uint32_t* vals;
-    uint32_t* gbegin;
-    uint32_t* gkey;
-    uint32_t* ghasrun;
-    int32_t* gsign;
-    int64_t n;
-    __device__ void flush(uint32_t gid, int32_t sg, bool run) const {
-        if (sg) atomicAdd(&gsign[gid], sg);
-        if (run) ghasrun[gid] = 1u;
+// Inclusive scan restarting at every lane with head set.
+__device__ inline int32_t seg_incl_scan(int32_t v, bool head) {
+    const int lane = lane_id();
+    int f = head ? 1 : 0;
+#pragma unroll
+    for (int d = 1; d < WAVE; d <<= 1) {
+        int32_t ov = __shfl_up(v, d, WAVE);
+        int of = __shfl_up(f, d, WAVE);
+        if (lane >= d && !f) v = ov + v;
+        if (lane >= d) f |= of;
     }
-    // items [base, base + SCAN_ITEMS) of flags v (1: a group starts), r = the
-    // groups started before base
-    __device__ void chunk(int64_t base, int64_t n_, uint32_t r, const uint32_t* v) const {
-        uint32_t gid = 0;
-        int32_t sg = 0;
-        bool run = false, open = false;
-        for (int j = 0; j < SCAN_ITEMS; j++) {
-            const int64_t i = base + j;
-            if (i >= n_) break;
-            if (v[j]) {
-                if (open) flush(gid, sg, run);
-                gid = r;
-                gbegin[gid] = (uint32_t)i;
-                gkey[gid] = keys[i];
-                sg = 0;
-                run = false;
-            } else if (!open) {
-                gid = r - 1;  // the group continues from the previous chunk
-            }
-            open = true;
-            r += v[j];
-            const uint32_t val = vals[i];
-            if (val >> 31)
-                sg += (int8_t)(val & 0xffu);
-            else
-                run = true;
-            if (i == n_ - 1) gbegin[gid + 1] = (uint32_t)n_;
+    return v;
+}
+
+// The crossing sign of an entry's value (0 for a run).
+__device__ inline int32_t entry_sign(uint32_t v) { return v >> 31 ? (int32_t)(int8_t)(v & 0xffu) : 0; }
+
+// Each tile row's entries among the sorted ones and its crossing sum, in one
+// pass over the entries.  A tile's entries are found again by the two tile
+// kernels, from the keys of the 64 entries that a wave has in hand: tables of the
+// distinct keys (their first entry, whether they hold a run, their crossing sum)
+// took a device-wide scan, two zeroed arrays and a pass of their own, 410 us for
+// the 20 million entries of 24 blobs against 36 us for this kernel.
+constexpr int RTAB_ITEMS = 8;  // entries per lane
+__global__ __launch_bounds__(256) void k_row_table(const uint32_t* keys, const uint32_t* vals, int64_t R,
+                                                   uint32_t xbits, uint32_t* row_begin, uint32_t* row_end,
+                                                   int32_t* row_sign) {
+    const int lane = lane_id();
+    const int64_t w = (int64_t)blockIdx.x * 4 + threadIdx.x / WAVE;
+    int64_t i = w * (WAVE * RTAB_ITEMS) + lane;
+    if (i - lane >= R) return;
+    uint32_t left = i - lane > 0 ? keys[i - lane - 1] >> xbits : 0xffffffffu;  // the row before the wave's next entry
+    uint32_t acc_row = 0;  // crossing sums of the row the last entries were in, per lane
+    int32_t acc = 0;
+    auto flush = [&]() {
+        for (int d = 32; d >= 1; d >>= 1) acc += __shfl_xor(acc, d, WAVE);
+        if (lane == 0 && acc) atomicAdd(&row_sign[acc_row], acc);
+        acc = 0;
+    };
+#pragma unroll
+    for (int k = 0; k < RTAB_ITEMS; k++, i += WAVE) {
+        if (i - lane >= R) break;
+        const bool valid = i < R;
+        const uint32_t row = valid ? keys[i] >> xbits : 0xfffffffeu;
+        const int32_t sg = valid ? entry_sign(vals[i]) : 0;
+        uint32_t prev = __shfl_up(row, 1, WAVE);
+        if (lane == 0) prev = left;
+        const bool head = valid && row != prev;
+        if (head) {
+            row_begin[row] = (uint32_t)i;
+            if (prev != 0xffffffffu) row_end[prev] = (uint32_t)i;
         }
-        if (open) flush(gid, sg, run);
+        if (i == R - 1) row_end[row] = (uint32_t)R;
+        const uint32_t r0 = __builtin_amdgcn_readfirstlane(row);
+        if (__ballot(valid && row != r0) == 0) {  // one row
+            if (r0 != acc_row) {
+                if (__ballot(acc != 0)) flush();
+                acc_row = r0;
+            }
+            acc += sg;
+        } else if (__ballot(sg != 0)) {
+            const int32_t sum = seg_incl_scan(sg, head || lane == 0);
+            const uint32_t next = __shfl_down(row, 1, WAVE);
+            if (valid && (lane == WAVE - 1 || next != row) && sum) atomicAdd(&row_sign[row], sum);
+        }
+        left = __shfl(row, WAVE - 1, WAVE);
     }
-};
-
-struct RowArgs {
-    const uint32_t* gkey;
-    const int32_t* gsign;
-    const uint32_t* n_groups;
-    uint32_t xbits;
-    uint32_t* row_gbegin;
-    uint32_t* row_gend;
-    int32_t* row_sign;
-};
-
-__global__ void k_row_table(RowArgs a, int64_t cap) {
-    const uint32_t G = *a.n_groups;
-    for (int64_t g = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; g < G && g < cap;
-         g += (int64_t)gridDim.x * blockDim.x) {
-        uint32_t row = a.gkey[g] >> a.xbits;
-        if (g == 0 || (a.gkey[g - 1] >> a.xbits) != row) a.row_gbegin[row] = (uint32_t)g;
-        if (g == G - 1 || (a.gkey[g + 1] >> a.xbits) != row) a.row_gend[row] = (uint32_t)g + 1;
-        int s = a.gsign[g];
-        if (s) atomicAdd(&a.row_sign[row], s);
-    }
+    if (__ballot(acc != 0)) flush();
 }
 
 // Per path: winding entering each tile row (the running sum of all earlier
@@ -744,7 +737,7 @@ __global__ void k_row_table(RowArgs a, int64_t cap) {
 // up to 600 rows against 14 now (10,000 paths of about 6 rows: 5.2 us).
 constexpr int PR_WAVES = 4;  // paths per workgroup
 __global__ __launch_bounds__(PR_WAVES * WAVE) void k_path_rows(const PathGrid* grid, int64_t n_paths,
-                                                               const uint32_t* row_gbegin, const uint32_t* row_gend,
+                                                               const uint32_t* row_begin, const uint32_t* row_end,
                                                                const int32_t* row_sign, int32_t* row_wb,
                                                                uint32_t* row_path, uint64_t* row_cnt) {
     const int lane = lane_id();
@@ -762,7 +755,7 @@ __global__ __launch_bounds__(PR_WAVES * WAVE) void k_path_rows(const PathGrid* g
             row_wb[row] = running + incl - v;
             row_path[row] = (uint32_t)p;
         }
-        nonempty |= __ballot(valid && row_gend[row] > row_gbegin[row]) != 0;
+        nonempty |= __ballot(valid && row_end[row] > row_begin[row]) != 0;
         running += __shfl(incl, WAVE - 1, WAVE);
     }
     if (lane == 0) {
@@ -777,16 +770,13 @@ __global__ __launch_bounds__(PR_WAVES * WAVE) void k_path_rows(const PathGrid* g
 struct TileArgs {
     const PathGrid* grid;
     const uint32_t* row_path;
-    const uint32_t* row_gbegin;
-    const uint32_t* row_gend;
+    const uint32_t* row_begin;  // the row's entries
+    const uint32_t* row_end;
     const int32_t* row_wb;
     int64_t n_rows;
-    const uint32_t* gbegin;
-    const uint32_t* gkey;
-    const uint32_t* ghasrun;
-    const int32_t* gsign;
+    const uint32_t* keys;     // sorted entries
+    const uint32_t* vals;
     uint32_t xbits;
-    const uint32_t* vals;     // sorted entry values
     const RunRec* recs;
     const float4* lines;
     uint64_t* row_cnt;        // count pass output
@@ -799,137 +789,171 @@ struct TileArgs {
     Counters* cnt;
 };
 
-constexpr int TG = 32;             // groups per chunk (one lane each)
-constexpr int ROWS_PER_WAVE = 8;   // tile rows per wave
+__device__ inline uint32_t rl(uint32_t v, int j) { return (uint32_t)__builtin_amdgcn_readlane((int)v, j); }
 
-// Inclusive scan restarting at every lane with head set.
-__device__ inline int32_t seg_incl_scan(int32_t v, bool head) {
-    const int lane = lane_id();
-    int f = head ? 1 : 0;
-#pragma unroll
-    for (int d = 1; d < WAVE; d <<= 1) {
-        int32_t ov = __shfl_up(v, d, WAVE);
-        int of = __shfl_up(f, d, WAVE);
-        if (lane >= d && !f) v = ov + v;
-        if (lane >= d) f |= of;
+// The bins (rasterizer.rs:193-213) of a tile row's sorted entries, 64 at a time,
+// one after another: the row's open bin and winding, and the previous tile.  All
+// of it is uniform.  step(key, vals of the wave's entries, n of them) calls
+// part(j0, j1) for each bin's entries that hold a run and tile(x) where a bin with
+// runs ends (after its last part), span(x, width) before it where the gap to the
+// previous tile is filled (rasterizer.rs:252-264).
+struct RowBins {
+    int32_t winding;       // after all entries so far
+    bool open = false, open_run = false, have_prev = false;
+    int32_t open_x = 0, open_w = 0;  // the open bin's x in the grid, the winding after its entries
+    int32_t prev_x = 0, prev_w = 0;
+
+    template <class Tile, class Span>
+    __device__ void close(Tile&& tile, Span&& span) {
+        if (open && open_run) {
+            if (have_prev && open_x > prev_x + 1 && prev_w != 0) span(prev_x + 1, open_x - prev_x - 1);
+            tile(open_x);
+            have_prev = true;
+            prev_x = open_x;
+            prev_w = open_w;
+        }
+        open = false;
     }
-    return v;
-}
+    template <class Part, class Tile, class Span>
+    __device__ void step(uint32_t key, uint32_t val, uint32_t n, uint32_t xmask, Part&& part, Tile&& tile,
+                         Span&& span) {
+        const int lane = lane_id();
+        const bool valid = (uint32_t)lane < n;
+        const uint64_t runs = __ballot(valid && !(val >> 31));
+        const uint32_t before = __shfl_up(key, 1, WAVE);
+        uint64_t heads = __ballot(valid && (lane == 0 || key != before));
+        int32_t wsum = valid ? entry_sign(val) : 0;
+        const bool cross = __ballot(wsum != 0) != 0;
+        if (cross) wsum = wave_incl_scan(wsum, OpAdd());
+        heads &= heads - 1;  // the starts after the first
+        uint32_t j0 = 0;
+        while (j0 < n) {
+            const uint32_t j1 = heads ? (uint32_t)__builtin_ctzll(heads) : n;
+            heads &= heads - 1;
+            const int32_t x = (int32_t)(rl(key, (int)j0) & xmask);
+            if (open && x != open_x) close(tile, span);
+            if (!open) {
+                open = true;
+                open_run = false;
+                open_x = x;
+            }
+            if (((runs >> j0) << (64u - (j1 - j0))) != 0) {
+                open_run = true;
+                part(j0, j1);
+            }
+            open_w = winding + (cross ? (int32_t)rl((uint32_t)wsum, (int)j1 - 1) : 0);
+            j0 = j1;
+        }
+        winding = open_w;
+    }
+};
 
-// Count pass of the tile stage: tiles and spans per tile row.  One wave per
-// block of 8 consecutive tile rows; each chunk of up to 32 groups is handled
-// one lane per group, the rows' running winding carried between chunks.
-__global__ __launch_bounds__(WAVE) void k_tile_counts(TileArgs a) {
-    // per row slot: running winding, tiles, spans, pending tile (for spans)
-    __shared__ int32_t r_w[ROWS_PER_WAVE], r_pend_tx[ROWS_PER_WAVE], r_pend_w[ROWS_PER_WAVE];
-    __shared__ uint32_t r_nt[ROWS_PER_WAVE], r_ns[ROWS_PER_WAVE], r_pend[ROWS_PER_WAVE];
-    const int lane = threadIdx.x;
+// Count pass of the tile stage: tiles and spans per tile row, one wave per row,
+// RowBins' rules with a lane per entry: a tile starts at the first run of a bin,
+// and the tile before it is the bin of the last run before the bin's entries (in
+// the wave's 64 entries, or carried from the ones before).  (RowBins here, bin
+// after bin in scalar code, measured 222 us against 143 on 24 blobs.)
+constexpr int TC_ROWS = 4;   // rows per workgroup
+constexpr int TC_AHEAD = 4;  // steps of 64 entries loaded ahead
+__global__ __launch_bounds__(TC_ROWS * WAVE) void k_tile_counts(TileArgs a) {
+    const int lane = lane_id();
     const uint64_t lt = lanemask_lt();
-    const uint64_t le = lane == 63 ? ~0ull : ((2ull << lane) - 1);
     const uint32_t xmask = (1u << a.xbits) - 1;
-    const int64_t n_blocks = (a.n_rows + ROWS_PER_WAVE - 1) / ROWS_PER_WAVE;
-    for (int64_t blk = blockIdx.x; blk < n_blocks; blk += gridDim.x) {
-        const int64_t R0 = blk * ROWS_PER_WAVE;
-        // lanes 0..7 describe the block's rows
-        uint32_t gb = 0xffffffffu, ge = 0;
-        bool real_row = false;
-        if (lane < ROWS_PER_WAVE && R0 + lane < a.n_rows) {
-            const int64_t row = R0 + lane;
-            const uint32_t p = a.row_path[row];
-            const PathGrid G = a.grid[p];
-            real_row = row - (int64_t)G.row_base < G.h;  // not the empty-path row
-            if (real_row) {
-                uint32_t b = a.row_gbegin[row], e = a.row_gend[row];
-                if (e > b) {
-                    gb = b;
-                    ge = e;
-                }
-                r_w[lane] = a.row_wb[row];
+    for (int64_t row = (int64_t)blockIdx.x * TC_ROWS + threadIdx.x / WAVE; row < a.n_rows;
+         row += (int64_t)gridDim.x * TC_ROWS) {
+        const PathGrid G = a.grid[a.row_path[row]];
+        if (row - (int64_t)G.row_base >= G.h) continue;  // the empty-path row (k_path_rows)
+        const uint32_t eb = __builtin_amdgcn_readfirstlane(a.row_begin[row]);
+        const uint32_t ee = __builtin_amdgcn_readfirstlane(a.row_end[row]);
+        int32_t winding = __builtin_amdgcn_readfirstlane(a.row_wb[row]);
+        uint32_t nt = 0, ns = 0;
+        // the last tile before the entries in hand, and the bin they may continue
+        bool have_prev = false, open_run = false;
+        int32_t prev_x = 0, prev_w = 0, open_x = -1;
+        auto load = [&](const uint32_t* p, uint32_t b, uint32_t none) {
+            return b + (uint32_t)lane < ee ? p[b + (uint32_t)lane] : none;
+        };
+        auto step = [&](uint32_t b, uint32_t key, uint32_t v) {
+            const int32_t x = (int32_t)(key & xmask);
+            const uint32_t n = min((uint32_t)WAVE, ee - b);
+            const bool valid = (uint32_t)lane < n, run = valid && !(v >> 31);
+            int32_t w = valid ? entry_sign(v) : 0;
+            w = winding + (__ballot(w != 0) ? wave_incl_scan(w, OpAdd()) : 0);
+            const int32_t left_x = __shfl_up(x, 1, WAVE);
+            const uint64_t heads = __ballot(valid && (lane == 0 || x != left_x)), runs = __ballot(run);
+            const int my = 63 - __clzll((long long)(heads & (lt | (1ull << lane))));  // the start of my bin's entries
+            // w after the bin that lane r's entry is in
+            auto bin_end = [&](int r) {
+                const uint64_t later = heads & (r == 63 ? 0ull : ~0ull << (r + 1));
+                return later ? (int)__builtin_ctzll(later) - 1 : (int)n - 1;
+            };
+            const bool cont = (int32_t)rl((uint32_t)x, 0) == open_x;  // the first bin continues the one before
+            const int32_t w0 = (int32_t)rl((uint32_t)w, bin_end(0));
+            if (open_run && !cont) {  // it has ended: the last tile
+                have_prev = true;
+                prev_x = open_x;
+                prev_w = winding;
             }
-            r_nt[lane] = 0;
-            r_ns[lane] = 0;
-            r_pend[lane] = 0;
-        }
-        uint32_t G0 = gb, G1 = ge;
+            const uint64_t below = (1ull << my) - 1ull;  // entries of earlier bins
+            const bool starts = run && (runs & lt & ~below) == 0 && !(my == 0 && cont && open_run);
+            const uint64_t before = runs & below;
+            const int r = before ? 63 - __clzll((long long)before) : 0;
+            const int32_t rx = __shfl(x, r, WAVE), rw = __shfl(w, bin_end(r), WAVE);
+            const bool from_open = my > 0 && cont && open_run;
+            const bool hp = before || from_open || have_prev;
+            const int32_t px = before ? rx : (from_open ? open_x : prev_x);
+            const int32_t pw = before ? rw : (from_open ? w0 : prev_w);
+            nt += (uint32_t)__popcll(__ballot(starts));
+            ns += (uint32_t)__popcll(__ballot(starts && hp && x > px + 1 && pw != 0));
+            // the last bin stays open; the last tile before it
+            const int last = (int)rl((uint32_t)my, (int)n - 1);
+            if (last > 0) {
+                const bool l_before = (runs & ((1ull << last) - 1ull)) != 0, l_open = cont && open_run;
+                prev_x = (int32_t)rl((uint32_t)px, (int)n - 1);
+                prev_w = (int32_t)rl((uint32_t)pw, (int)n - 1);
+                have_prev = l_before || l_open || have_prev;
+            }
+            open_run = (runs >> last) != 0 || (last == 0 && cont && open_run);
+            open_x = (int32_t)rl((uint32_t)x, (int)n - 1);
+            winding = (int32_t)rl((uint32_t)w, (int)n - 1);
+        };
+        // TC_AHEAD steps' entries loaded together, the next ones while they are taken
+        uint32_t key[TC_AHEAD], val[TC_AHEAD];
+        auto load_all = [&](uint32_t b) {
 #pragma unroll
-        for (int d = 1; d < ROWS_PER_WAVE; d <<= 1) {
-            G0 = min(G0, (uint32_t)__shfl_xor(G0, d, WAVE));
-            G1 = max(G1, (uint32_t)__shfl_xor(G1, d, WAVE));
-        }
-        G0 = __shfl(G0, 0, WAVE);
-        G1 = __shfl(G1, 0, WAVE);
-        __syncthreads();
-        for (uint32_t c = G0; c < G1 && G0 < G1; c += TG) {
-            const uint32_t g = c + lane;
-            const bool valid = lane < TG && g < G1;
-            const uint32_t key = valid ? a.gkey[g] : 0u;
-            const int64_t row = (int64_t)(key >> a.xbits);
-            const int slot = valid ? (int)(row - R0) : ROWS_PER_WAVE;
-            int32_t tx = 0;
-            if (valid) {
-                const PathGrid G = a.grid[a.row_path[row]];
-                tx = G.tx0 + (int32_t)(key & xmask);
+            for (int k = 0; k < TC_AHEAD; k++) {
+                key[k] = load(a.keys, b + (uint32_t)(k * WAVE), 0u);
+                val[k] = load(a.vals, b + (uint32_t)(k * WAVE), 0x80000000u);
             }
-            const bool hr = valid && a.ghasrun[g];
-            const int32_t sg = valid ? a.gsign[g] : 0;
-            const int prev_slot = __shfl_up(slot, 1, WAVE);
-            const bool head = lane == 0 || prev_slot != slot;
-            // lanes of my row slot
-            uint64_t same = __ballot(valid);
+        };
+        load_all(eb);
+        for (uint32_t b = eb; b < ee; b += TC_AHEAD * WAVE) {
+            uint32_t ck[TC_AHEAD], cv[TC_AHEAD];
 #pragma unroll
-            for (int b = 0; b < 4; b++) {
-                const bool bit = (slot >> b) & 1;
-                const uint64_t m = __ballot(bit);
-                same &= bit ? m : ~m;
+            for (int k = 0; k < TC_AHEAD; k++) {
+                ck[k] = key[k];
+                cv[k] = val[k];
             }
-            const uint64_t tiles = __ballot(hr);
-            const int32_t wend = (valid ? r_w[slot] : 0) + seg_incl_scan(sg, head);
-            const uint64_t my_tiles = tiles & same;
-            // spans to the next tile of the same row (rasterizer.rs:252-264)
-            const uint64_t above = my_tiles & ~le;
-            const int nb = above ? (__ffsll((long long)above) - 1) : lane;
-            const int32_t btx = __shfl(tx, nb, WAVE);
-            const bool span_here = hr && above && btx > tx + 1 && wend != 0;
-            // the first tile of a row in this chunk closes that row's pending tile
-            const bool first_tile = hr && (my_tiles & lt) == 0;
-            bool pend_span = false;
-            if (first_tile && r_pend[slot]) pend_span = tx > r_pend_tx[slot] + 1 && r_pend_w[slot] != 0;
-            const uint64_t spans = __ballot(span_here);
-            const uint64_t pends = __ballot(pend_span);
-            __syncthreads();
-            // per-row state after this chunk: the last lane of each row segment
-            const int next_slot = __shfl_down(slot, 1, WAVE);
-            const bool tail = valid && (lane == WAVE - 1 || next_slot != slot || !(lane + 1 < TG && c + lane + 1 < G1));
-            const int last = my_tiles ? 63 - __clzll((long long)my_tiles) : lane;
-            const int32_t ltx = __shfl(tx, last, WAVE);
-            const int32_t lw = __shfl(wend, last, WAVE);
-            if (tail) {
-                r_w[slot] = wend;
-                r_nt[slot] += (uint32_t)__popcll(my_tiles);
-                r_ns[slot] += (uint32_t)__popcll(spans & same) + (uint32_t)__popcll(pends & same);
-                if (my_tiles) {
-                    r_pend[slot] = 1;
-                    r_pend_tx[slot] = ltx;
-                    r_pend_w[slot] = lw;
-                }
-            }
-            __syncthreads();
+            load_all(b + TC_AHEAD * WAVE);
+#pragma unroll
+            for (int k = 0; k < TC_AHEAD; k++)
+                if (b + (uint32_t)(k * WAVE) < ee) step(b + (uint32_t)(k * WAVE), ck[k], cv[k]);
         }
-        if (lane < ROWS_PER_WAVE && R0 + lane < a.n_rows && real_row)
-            a.row_cnt[R0 + lane] = ((uint64_t)r_nt[lane] << 32) | r_ns[lane];
-        __syncthreads();
+        if (lane == 0) a.row_cnt[row] = ((uint64_t)nt << 32) | ns;
     }
 }
 
 // Emit pass of the tile stage: one wave per tile row, walking the row's
-// groups (bins, rasterizer.rs:213-265) in key order.  The row's sort entries
+// bins (rasterizer.rs:213-265) in key order.  The row's sort entries
 // are taken TR_BLOCK at a time and each lane replays one run into LDS: its
-// increments in step order, its first pixel, and its bit in the `hit` words of
-// the pixels it visits.  A run stays inside one 8x8 tile and its walk moves one
-// pixel along one axis per step, so it has at most 15 increments, at distinct
-// pixels, and the increment at a pixel is the one whose step is the pixel's
-// distance |dx| + |dy| from the run's first pixel: no map from pixel to step is
-// needed.  Each lane then owns a pixel of the tile and adds, for the set bits of
+// increments, and its bit in the `hit` words of the pixels it visits.  A run stays
+// inside one 8x8 tile and its walk moves one pixel along one axis per step, always
+// in the same direction along that axis, so it has at most 15 increments, at
+// distinct pixels, and along it x + y (its directions along x and y alike) or
+// x - y (unlike) moves by one per step: that is the increment's slot, which a pixel
+// knows of itself, given the run's bit in the block's mask of alike ones.  No map
+// from pixel to step is kept or read.  Each lane then owns a pixel of the tile and
+// adds, for the set bits of
 // its hit words among the tile's runs, in sorted order, the increments found
 // there to its register sums, so every pixel's f32 sums follow the sorted order
 // exactly (rasterizer.rs:221-228), with no read-modify-write through LDS.  At
@@ -946,13 +970,11 @@ __global__ __launch_bounds__(WAVE) void k_tile_counts(TileArgs a) {
 // 4, instead of its runs, about 11), the next block's records and lines load
 // while this one is added, and the carry moves by DPP instead of eight LDS
 // permutes.
-// Measured against the 32-run kernel with maps: 120 -> 45 us on a line of 61
-// glyphs, 422 -> 220 us on 10,000 glyphs, 2,684 -> 1,000 us on 24 star blobs of
-// 1,000-20,000 cubics.
+// Measured against the 32-run kernel with maps: 120 -> 43 us on a line of 61
+// glyphs, 422 -> 203 us on 10,000 glyphs (81% of the SIMDs' VALU cycles), 2,684 ->
+// 930 us on 24 star blobs of 1,000-20,000 cubics.
 constexpr int TR_SLOTS = 15;  // increments per run
 constexpr int TR_BLOCK = WAVE;  // runs replayed per block
-
-__device__ inline uint32_t rl(uint32_t v, int j) { return (uint32_t)__builtin_amdgcn_readlane((int)v, j); }
 
 // The first tile row of a workgroup of a row kernel (rows first_row +
 // k * gridDim.x).  Neighbouring tile rows gather the same lines and run
@@ -974,12 +996,12 @@ static inline uint32_t row_grid(int64_t rows, int64_t cap) {
 }
 
 // The increments of a run from the DDA state at its first one (p0: that
-// increment's start point) into `inc` in step order, and the run's bit into the
-// hit words of its pixels; CARRY: every active lane's line is finite, so each
+// increment's start point) into their slots from inc[0] on, `dir` apart, and the
+// run's bit into the hit words of its pixels; CARRY: every active lane's line is finite, so each
 // increment's start point is the previous one's end point (see
 // dda_increment_carried).
 template <bool CARRY>
-__device__ inline void tr_replay_steps(float2* inc, uint32_t* hit, uint32_t bit, Dda& d, V2 p0, bool finite,
+__device__ inline void tr_replay_steps(float2* inc, int dir, uint32_t* hit, uint32_t bit, Dda& d, V2 p0, bool finite,
                                        Counters* cnt) {
     uint32_t lx = (uint32_t)(d.x & 7), ly = (uint32_t)(d.y & 7);
     const uint32_t lxd = (uint32_t)(int32_t)d.x_dir, lyd = (uint32_t)(int32_t)d.y_dir;
@@ -987,7 +1009,8 @@ __device__ inline void tr_replay_steps(float2* inc, uint32_t* hit, uint32_t bit,
     for (int k = 0; k < TR_SLOTS; k++) {
         float area, height;
         dda_increment_carried(d, p0, CARRY || finite, area, height);
-        inc[k] = make_float2(area, height);
+        *inc = make_float2(area, height);
+        inc += dir;
         atomicOr(&hit[(ly << 3) | lx], bit);
         // dda_step, with the in-tile pixel moved alongside
         float c;
@@ -1011,151 +1034,73 @@ __device__ inline void tr_replay_steps(float2* inc, uint32_t* hit, uint32_t bit,
     if (!ended) atomicOr(&cnt->error, (uint32_t)ERR_REPLAY);
 }
 
-// The lane's value of v from DPP_CTRL's source lane; `old` where there is none.
-template <int DPP_CTRL>
+template <int CTRL>
 __device__ inline float dpp_f(float old, float v) {
-    return __int_as_float(
-        __builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(v), DPP_CTRL, 0xf, 0xf, false));
+    return __uint_as_float(dpp<CTRL>(__float_as_uint(old), __float_as_uint(v)));
 }
-constexpr int DPP_ROW_SHR2 = 0x112, DPP_ROW_ROR2 = 0x122;  // within each 16 lanes
 
 __global__ __launch_bounds__(WAVE) void k_tile_rows(TileArgs a) {
     __shared__ float2 inc[TR_BLOCK * TR_SLOTS];
-    __shared__ uint32_t hit[2][64];        // pixel p, bit j: run 32 w + j visits p
-    __shared__ uint16_t first[TR_BLOCK];   // a run's first pixel, x | y << 8
+    __shared__ uint32_t hit[2][64];  // pixel p, bit j: run 32 w + j visits p
     const int lane = threadIdx.x;
     // Lane -> pixel: 16 lanes hold two pixel rows interleaved, so that a move of
     // two lanes is the next pixel of the same row and the first two lanes, which
     // have no source, keep the carry.
     const uint32_t px = (uint32_t)(lane >> 1) & 7u, py = (uint32_t)((lane >> 4) << 1) | (uint32_t)(lane & 1);
-    const uint32_t pix = (py << 3) | px, pos = px | (py << 8);
+    const uint32_t pix = (py << 3) | px, slot_alike = px + py, slot_unlike = px + 7u - py;
     const uint32_t xmask = (1u << a.xbits) - 1;
     for (int64_t row = xcd_first_row(); row < a.n_rows; row += gridDim.x) {
         const PathGrid G = a.grid[a.row_path[row]];
         if (row - (int64_t)G.row_base >= G.h) continue;  // the empty-path row (k_path_out)
-        const uint32_t gb = a.row_gbegin[row], ge = a.row_gend[row];
-        if (ge <= gb) continue;
+        const uint32_t eb = __builtin_amdgcn_readfirstlane(a.row_begin[row]);
+        const uint32_t ee = __builtin_amdgcn_readfirstlane(a.row_end[row]);
+        if (ee <= eb) continue;
         const int32_t ty = G.ty0 + (int32_t)(row - (int64_t)G.row_base);
         const uint64_t off = a.row_off[row];
         const uint32_t row_tiles = (uint32_t)(off >> 32), row_spans = (uint32_t)off;
-        const uint32_t E_hi = a.gbegin[ge];
-        int32_t winding = a.row_wb[row];
+        RowBins bins;
+        bins.winding = __builtin_amdgcn_readfirstlane(a.row_wb[row]);
         float carry = 0.0f;  // of the lane's pixel row, in its first lane
         uint32_t nt = 0, ns = 0;
-        bool have_prev = false;
-        int32_t prev_tx = 0, prev_w = 0;
-        // groups gbase + lane: key, has runs, crossing sum, end of its entries
-        uint32_t gbase = gb, gk = 0, ghr = 0, gend = 0;
-        int32_t gsg = 0;
-        auto load_groups = [&]() {
-            const uint32_t g = gbase + (uint32_t)lane;
-            if (g < ge) {
-                gk = a.gkey[g];
-                ghr = a.ghasrun[g];
-                gsg = a.gsign[g];
-                gend = a.gbegin[g + 1];
-            }
-        };
-        load_groups();
-        uint32_t e = a.gbegin[gb];
-        // the block after the current one: its entries' values, records and lines
-        auto load_val = [&](uint32_t base) {
-            const uint32_t ei = base + (uint32_t)lane;
-            return ei < E_hi ? a.vals[ei] : 0x80000000u;
-        };
-        auto load_rec = [&](uint32_t v) { return v >> 31 ? RunRec{0, 0, 0.0f, 0.0f} : a.recs[v]; };
-        auto load_line = [&](uint32_t v, const RunRec& r) {
-            return v >> 31 ? make_float4(0, 0, 0, 0) : a.lines[r.line & 0x7fffffffu];
-        };
-        uint32_t nv = load_val(e);
-        RunRec nr = load_rec(nv);
-        float4 nl = load_line(nv, nr);
-        uint32_t nv2 = load_val(e + TR_BLOCK);
-        uint32_t next = e, ebase = 0;     // first entry of the next and of the current block
-        uint32_t h0 = 0, h1 = 0;          // this pixel's hit words of the current block
-        float pa = 0.0f, ph = 0.0f;       // this pixel's sums of the current tile
-        for (uint32_t g = gb; g < ge; g++) {
-            if (g - gbase >= (uint32_t)WAVE) {
-                gbase = g;
-                load_groups();
-            }
-            const int j = (int)(g - gbase);
-            const uint32_t key = rl(gk, j), hr = rl(ghr, j), g_end = rl(gend, j);
-            winding += (int32_t)rl((uint32_t)gsg, j);
-            if (!hr) {  // tile-row crossings only (a block's entries are taken in order all the same)
-                e = g_end;
-                continue;
-            }
-            const int32_t tx = G.tx0 + (int32_t)(key & xmask);
-            if (have_prev && tx > prev_tx + 1 && prev_w != 0) {
-                if (lane == 0) {
-                    const uint32_t si = row_spans + ns;
-                    a.span_xy[2 * si] = (int16_t)((prev_tx + 1) * TILE);
-                    a.span_xy[2 * si + 1] = (int16_t)(ty * TILE);
-                    a.span_w[si] = (uint16_t)((uint16_t)(tx - prev_tx - 1) * (uint16_t)TILE);
+        float pa = 0.0f, ph = 0.0f;  // this pixel's sums of the open tile
+        uint32_t h0 = 0, h1 = 0;     // this pixel's hit words of the block
+        uint64_t alike = 0;          // the block's runs whose slots are x + y
+        // two hits at a time: their reads are in flight together
+        auto add_runs = [&](uint32_t h, uint32_t al, uint32_t lo, uint32_t hi, const float2* incs) {
+            uint32_t m = h & (0xffffffffu << lo) & (0xffffffffu >> (32u - hi));
+            auto at = [&](uint32_t r) {
+                return incs[r * (uint32_t)TR_SLOTS + ((al >> r) & 1u ? slot_alike : slot_unlike)];
+            };
+            while (m) {
+                const uint32_t r1 = (uint32_t)__ffs((int)m) - 1u;
+                m &= m - 1u;
+                const uint32_t r2 = m ? (uint32_t)__ffs((int)m) - 1u : r1;
+                const float2 v1 = at(r1), v2 = at(r2);
+                pa = pa + v1.x;
+                ph = ph + v1.y;
+                if (m) {
+                    pa = pa + v2.x;
+                    ph = ph + v2.y;
                 }
-                ns++;
+                m &= m - 1u;
             }
-            while (e < g_end) {
-                while (e >= next) {
-                    // (c) replay the next TR_BLOCK entries, one run per lane
-                    ebase = next;
-                    next += TR_BLOCK;
-                    const uint32_t v = nv;
-                    const RunRec r = nr;
-                    const float4 L = nl;
-                    nv = nv2;
-                    nr = load_rec(nv);
-                    __syncthreads();  // the previous block's increments are read
-                    hit[0][lane] = 0;
-                    hit[1][lane] = 0;
-                    __syncthreads();
-                    if (!(v >> 31)) {
-                        Dda d;
-                        const V2 last = mk(L.x, L.y), point = mk(L.z, L.w);
-                        if (r.line >> 31) {
-                            dda_init(d, last, point);
-                        } else {
-                            dda_consts(d, last, point);
-                            d.x = (int16_t)(r.xy & 0xffffu);
-                            d.y = (int16_t)(r.xy >> 16);
-                            d.row_t1 = r.row_t1;
-                            d.col_t1 = r.col_t1;
-                            d.t0 = 0.0f;
-                            dda_step(d);
-                        }
-                        const bool finite = line_finite(last, point);
-                        const V2 p0 = dda_point(d, d.t0);
-                        first[lane] = (uint16_t)((d.x & 7) | ((d.y & 7) << 8));
-                        float2* out = inc + lane * TR_SLOTS;
-                        uint32_t* hw = hit[lane >> 5];
-                        const uint32_t bit = 1u << (lane & 31);
-                        if (__ballot(!finite) == 0) tr_replay_steps<true>(out, hw, bit, d, p0, finite, a.cnt);
-                        else tr_replay_steps<false>(out, hw, bit, d, p0, finite, a.cnt);
-                    }
-                    nl = load_line(nv, nr);
-                    nv2 = load_val(next + TR_BLOCK);
-                    __syncthreads();
-                    h0 = hit[0][pix];
-                    h1 = hit[1][pix];
-                }
-                // the tile's runs of this block, added in sorted order
-                const uint32_t j0 = e - ebase, j1 = min(g_end, next) - ebase;
-                auto add_runs = [&](uint32_t h, uint32_t lo, uint32_t hi, const uint16_t* fst, const float2* incs) {
-                    uint32_t m = h & (0xffffffffu << lo) & (0xffffffffu >> (32u - hi));
-                    while (m) {
-                        const uint32_t r = (uint32_t)__ffs((int)m) - 1u;
-                        m &= m - 1u;
-                        // |dx| + |dy| from the run's first pixel, by bytes
-                        const float2 v = incs[__builtin_amdgcn_sad_u8((uint32_t)fst[r], pos, r * (uint32_t)TR_SLOTS)];
-                        pa = pa + v.x;
-                        ph = ph + v.y;
-                    }
-                };
-                if (j0 < 32u) add_runs(h0, j0, min(j1, 32u), first, inc);
-                if (j1 > 32u) add_runs(h1, j0 > 32u ? j0 - 32u : 0u, j1 - 32u, first + 32, inc + 32 * TR_SLOTS);
-                e = ebase + j1;
+        };
+        // a bin's runs of this block, added in sorted order
+        auto part = [&](uint32_t j0, uint32_t j1) {
+            if (j0 < 32u) add_runs(h0, (uint32_t)alike, j0, min(j1, 32u), inc);
+            if (j1 > 32u)
+                add_runs(h1, (uint32_t)(alike >> 32), j0 > 32u ? j0 - 32u : 0u, j1 - 32u, inc + 32 * TR_SLOTS);
+        };
+        auto span = [&](int32_t x, int32_t w) {
+            if (lane == 0) {
+                const uint32_t si = row_spans + ns;
+                a.span_xy[2 * si] = (int16_t)((G.tx0 + x) * TILE);
+                a.span_xy[2 * si + 1] = (int16_t)(ty * TILE);
+                a.span_w[si] = (uint16_t)((uint16_t)w * (uint16_t)TILE);
             }
+            ns++;
+        };
+        auto tile = [&](int32_t x) {
             // (d)(e) the fold along each pixel row: after k moves the lanes of
             // pixels 0..k hold ((carry + h0) + h1) ..., the later ones not yet
             float mine = carry, t = carry + ph;
@@ -1172,14 +1117,80 @@ __global__ __launch_bounds__(WAVE) void k_tile_rows(TileArgs a) {
             pa = 0.0f;
             ph = 0.0f;
             if (lane == 0) {
-                a.tile_xy[2 * ti] = (int16_t)(tx * TILE);
+                a.tile_xy[2 * ti] = (int16_t)((G.tx0 + x) * TILE);
                 a.tile_xy[2 * ti + 1] = (int16_t)(ty * TILE);
             }
             nt++;
-            have_prev = true;
-            prev_tx = tx;
-            prev_w = winding;
+        };
+        // the entries of a block, their records and lines
+        auto load = [&](const uint32_t* p, uint32_t b, uint32_t none) {
+            return b + (uint32_t)lane < ee ? p[b + (uint32_t)lane] : none;
+        };
+        auto load_rec = [&](uint32_t v) {  // (bit 31 of its line: the line's first run)
+            if ((v >> 30) == 1u) return a.recs[v & (RT_REC - 1u)];
+            return RunRec{v | 0x80000000u, 0, 0.0f, 0.0f};
+        };
+        auto load_line = [&](uint32_t v, const RunRec& r) {
+            return v >> 31 ? make_float4(0, 0, 0, 0) : a.lines[r.line & 0x7fffffffu];
+        };
+        // each level of a block's loads has a block's time: entries three blocks
+        // ahead, records two, lines one
+        uint32_t k1 = load(a.keys, eb, 0u), v1 = load(a.vals, eb, 0x80000000u);
+        uint32_t k2 = load(a.keys, eb + TR_BLOCK, 0u), v2 = load(a.vals, eb + TR_BLOCK, 0x80000000u);
+        uint32_t k3 = load(a.keys, eb + 2 * TR_BLOCK, 0u), v3 = load(a.vals, eb + 2 * TR_BLOCK, 0x80000000u);
+        RunRec r1 = load_rec(v1), r2 = load_rec(v2);
+        float4 l1 = load_line(v1, r1);
+        for (uint32_t b = eb; b < ee; b += TR_BLOCK) {
+            // (c) replay the block's entries, one run per lane
+            const uint32_t key = k1, v = v1;
+            const RunRec r = r1;
+            const float4 L = l1;
+            k1 = k2;
+            v1 = v2;
+            r1 = r2;
+            l1 = load_line(v1, r1);
+            k2 = k3;
+            v2 = v3;
+            r2 = load_rec(v2);
+            k3 = load(a.keys, b + 3 * TR_BLOCK, 0u);
+            v3 = load(a.vals, b + 3 * TR_BLOCK, 0x80000000u);
+            __syncthreads();  // the previous block's increments are read
+            hit[0][lane] = 0;
+            hit[1][lane] = 0;
+            __syncthreads();
+            bool al = false;
+            if (!(v >> 31)) {
+                Dda d;
+                const V2 last = mk(L.x, L.y), point = mk(L.z, L.w);
+                if (r.line >> 31) {
+                    dda_init(d, last, point);
+                } else {
+                    dda_consts(d, last, point);
+                    d.x = (int16_t)(r.xy & 0xffffu);
+                    d.y = (int16_t)(r.xy >> 16);
+                    d.row_t1 = r.row_t1;
+                    d.col_t1 = r.col_t1;
+                    d.t0 = 0.0f;
+                    dda_step(d);
+                }
+                const bool finite = line_finite(last, point);
+                const V2 p0 = dda_point(d, d.t0);
+                // (a direction is 0 only where a coordinate is not finite: that axis takes no step)
+                al = d.x_dir == d.y_dir || d.x_dir == 0 || d.y_dir == 0;
+                const int dir = d.x_dir ? d.x_dir : d.y_dir;
+                float2* out = inc + lane * TR_SLOTS + (al ? (d.x & 7) + (d.y & 7) : (d.x & 7) + 7 - (d.y & 7));
+                uint32_t* hw = hit[lane >> 5];
+                const uint32_t bit = 1u << (lane & 31);
+                if (__ballot(!finite) == 0) tr_replay_steps<true>(out, dir, hw, bit, d, p0, finite, a.cnt);
+                else tr_replay_steps<false>(out, dir, hw, bit, d, p0, finite, a.cnt);
+            }
+            __syncthreads();
+            h0 = hit[0][pix];
+            h1 = hit[1][pix];
+            alike = __ballot(al);
+            bins.step(key, v, min((uint32_t)TR_BLOCK, ee - b), xmask, part, tile, span);
         }
+        bins.close(tile, span);
     }
 }
 
@@ -1905,7 +1916,6 @@ static int run_plain_pass(Context* ctx, const SegInput& in, OutputDesc& out, hip
     da.xbits = 0;
     da.keys = da.vals = nullptr;
     da.recs = nullptr;
-    da.unordered = unordered;
     const int64_t nblk = (int64_t)grid_for(std::max<int64_t>(L, 1), 256);
     HIPCHK(ctx->dda_blk.ensure((size_t)nblk * 16));
     da.blk_entries = ctx->dda_blk.as<uint64_t>();
@@ -2088,54 +2098,33 @@ static int run_plain_pass(Context* ctx, const SegInput& in, OutputDesc& out, hip
     const uint32_t* skeys = ctx->keys[cur].as<uint32_t>();
     const uint32_t* svals = ctx->vals[cur].as<uint32_t>();
 
-    // ---- groups (one per distinct key) and tile rows
-    HIPCHK(ctx->grp_begin.ensure((std::max<int64_t>(R, 1) + 1) * 4));
-    HIPCHK(ctx->grp_key.ensure(std::max<int64_t>(R, 1) * 4));
-    HIPCHK(ctx->grp_hasrun.ensure(std::max<int64_t>(R, 1) * 4));
-    HIPCHK(ctx->grp_sign.ensure(std::max<int64_t>(R, 1) * 4));
-    fill<uint32_t>(ctx->grp_hasrun.as<uint32_t>(), R, 0u, s);
-    fill<int32_t>(ctx->grp_sign.as<int32_t>(), R, 0, s);
-    if (R > 0) {
-        HIPCHK(launch_scan<uint32_t>(ctx, R, LoadGroupStart{skeys},
-                                     StoreGroup{skeys, svals, ctx->grp_begin.as<uint32_t>(),
-                                                ctx->grp_key.as<uint32_t>(), ctx->grp_hasrun.as<uint32_t>(),
-                                                ctx->grp_sign.as<int32_t>(), R},
-                                     OpAdd(), 0u, reinterpret_cast<uint32_t*>(&tot[3]), s));
-    }
-    HIPCHK(ctx->row_gbegin.ensure(ROWS * 4));
-    HIPCHK(ctx->row_gend.ensure(ROWS * 4));
+    // ---- tile rows
+    HIPCHK(ctx->row_begin.ensure(ROWS * 4));
+    HIPCHK(ctx->row_end.ensure(ROWS * 4));
     HIPCHK(ctx->row_sign.ensure(ROWS * 4));
     HIPCHK(ctx->row_wb.ensure(ROWS * 4));
     HIPCHK(ctx->row_path.ensure(ROWS * 4));
     HIPCHK(ctx->row_cnt.ensure(ROWS * 8));
     HIPCHK(ctx->row_off.ensure(ROWS * 8));
-    fill<uint32_t>(ctx->row_gbegin.as<uint32_t>(), ROWS, 0u, s);
-    fill<uint32_t>(ctx->row_gend.as<uint32_t>(), ROWS, 0u, s);
+    uint32_t* row_begin = ctx->row_begin.as<uint32_t>();
+    uint32_t* row_end = ctx->row_end.as<uint32_t>();
+    fill<uint32_t>(row_begin, ROWS, 0u, s);
+    fill<uint32_t>(row_end, ROWS, 0u, s);
     fill<int32_t>(ctx->row_sign.as<int32_t>(), ROWS, 0, s);
-    RowArgs ra;
-    ra.gkey = ctx->grp_key.as<uint32_t>();
-    ra.gsign = ctx->grp_sign.as<int32_t>();
-    ra.n_groups = reinterpret_cast<const uint32_t*>(&tot[3]);
-    ra.xbits = xbits;
-    ra.row_gbegin = ctx->row_gbegin.as<uint32_t>();
-    ra.row_gend = ctx->row_gend.as<uint32_t>();
-    ra.row_sign = ctx->row_sign.as<int32_t>();
     if (R > 0)
-        hipLaunchKernelGGL(k_row_table, dim3(std::min<uint32_t>(grid_for(R, 256), 16384)), dim3(256), 0, s, ra, R);
-    hipLaunchKernelGGL(k_path_rows, dim3(grid_for(NP, PR_WAVES)), dim3(PR_WAVES * WAVE), 0, s, grid, NP, ra.row_gbegin, ra.row_gend,
-                       ra.row_sign, ctx->row_wb.as<int32_t>(), ctx->row_path.as<uint32_t>(),
+        hipLaunchKernelGGL(k_row_table, dim3(grid_for(R, 256 * RTAB_ITEMS)), dim3(256), 0, s, skeys, svals, R, xbits,
+                           row_begin, row_end, ctx->row_sign.as<int32_t>());
+    hipLaunchKernelGGL(k_path_rows, dim3(grid_for(NP, PR_WAVES)), dim3(PR_WAVES * WAVE), 0, s, grid, NP, row_begin,
+                       row_end, ctx->row_sign.as<int32_t>(), ctx->row_wb.as<int32_t>(), ctx->row_path.as<uint32_t>(),
                        ctx->row_cnt.as<uint64_t>());
     TileArgs ta;
     ta.grid = grid;
     ta.row_path = ctx->row_path.as<uint32_t>();
-    ta.row_gbegin = ra.row_gbegin;
-    ta.row_gend = ra.row_gend;
+    ta.row_begin = row_begin;
+    ta.row_end = row_end;
     ta.row_wb = ctx->row_wb.as<int32_t>();
     ta.n_rows = ROWS;
-    ta.gbegin = ctx->grp_begin.as<uint32_t>();
-    ta.gkey = ra.gkey;
-    ta.ghasrun = ctx->grp_hasrun.as<uint32_t>();
-    ta.gsign = ra.gsign;
+    ta.keys = skeys;
     ta.xbits = xbits;
     ta.vals = svals;
     ta.recs = ctx->records.as<RunRec>();
@@ -2148,8 +2137,8 @@ static int run_plain_pass(Context* ctx, const SegInput& in, OutputDesc& out, hip
     ta.span_xy = out.span_xy;
     ta.span_w = out.span_w;
     ta.cnt = cnt;
-    const uint32_t tile_blocks = (uint32_t)std::min<int64_t>((ROWS + ROWS_PER_WAVE - 1) / ROWS_PER_WAVE, 1 << 20);
-    hipLaunchKernelGGL(k_tile_counts, dim3(tile_blocks), dim3(WAVE), 0, s, ta);
+    const uint32_t tile_blocks = (uint32_t)std::min<int64_t>((ROWS + TC_ROWS - 1) / TC_ROWS, 1 << 20);
+    hipLaunchKernelGGL(k_tile_counts, dim3(tile_blocks), dim3(TC_ROWS * WAVE), 0, s, ta);
     HIPCHK(launch_scan<uint64_t>(ctx, ROWS, LoadU64{ta.row_cnt}, StoreU64{ctx->row_off.as<uint64_t>()}, OpAdd(),
                                  0ull, &tot[4], s));
     HIPCHK(hipGetLastError());
