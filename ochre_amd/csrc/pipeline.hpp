@@ -116,7 +116,8 @@ constexpr int64_t PLAIN_MAX_ENTRIES = 1ll << 30;
 
 struct Context {
     int device = 0;
-    hipStream_t own_stream = nullptr;
+    hipStream_t own_stream = nullptr;  // beside the caller's, within one call
+    hipEvent_t side_ev[2] = {nullptr, nullptr};
     // tile sums of the device-wide scans
     DBuf scan_partials;
     // pipeline scratch
@@ -126,7 +127,7 @@ struct Context {
     DBuf counters, totals;
     DBuf call_error;  // emit-phase error bits of the current plain call (all passes)
     DBuf keys[2], vals[2], records, rs_counts;
-    DBuf row_begin, row_end, row_sign, row_wb, row_path, row_cnt, row_off;
+    DBuf row_begin, row_end, long_rows, row_sign, row_wb, row_path, row_cnt, row_off;
     DBuf split_off;  // rebased per-path offsets of a path range (run_plain's split)
     DBuf u_pwbase, u_rwbase, u_bcnt, u_bbeg, u_bcur;  // unordered tile stage: window buckets
     double split_ratio = 2.0;  // how far the last pass that had to split was over its limits

@@ -65,6 +65,8 @@ Context::~Context() {
     if (host_pinned) (void)hipHostFree(host_pinned);
     for (auto& e : ev)
         if (e) (void)hipEventDestroy(e);
+    for (auto& e : side_ev)
+        if (e) (void)hipEventDestroy(e);
     if (own_stream) (void)hipStreamDestroy(own_stream);
 }
 
@@ -781,6 +783,8 @@ struct TileArgs {
     const float4* lines;
     uint64_t* row_cnt;        // count pass output
     const uint64_t* row_off;  // emit pass input: (tiles << 32) | spans exclusive offsets
+    uint32_t* long_rows;      // count pass output: the longest rows from the front, other long ones from the back
+    uint32_t* n_long;         // [0] longest, [1] other long
     int16_t* tile_xy;
     uint8_t* tile_alpha;
     float* tile_cov;          // optional pre-quantisation coverage, 64 per tile
@@ -854,6 +858,7 @@ struct RowBins {
 // the wave's 64 entries, or carried from the ones before).  (RowBins here, bin
 // after bin in scalar code, measured 222 us against 143 on 24 blobs.)
 constexpr int TC_ROWS = 4;   // rows per workgroup
+constexpr uint32_t TR_LONG = 32 * WAVE, TR_LONGEST = 96 * WAVE;  // entries of a long row (see k_tile_rows)
 constexpr int TC_AHEAD = 4;  // steps of 64 entries loaded ahead
 __global__ __launch_bounds__(TC_ROWS * WAVE) void k_tile_counts(TileArgs a) {
     const int lane = lane_id();
@@ -939,7 +944,11 @@ __global__ __launch_bounds__(TC_ROWS * WAVE) void k_tile_counts(TileArgs a) {
             for (int k = 0; k < TC_AHEAD; k++)
                 if (b + (uint32_t)(k * WAVE) < ee) step(b + (uint32_t)(k * WAVE), ck[k], cv[k]);
         }
-        if (lane == 0) a.row_cnt[row] = ((uint64_t)nt << 32) | ns;
+        if (lane == 0) {
+            a.row_cnt[row] = ((uint64_t)nt << 32) | ns;
+            if (ee - eb >= TR_LONGEST) a.long_rows[atomicAdd(&a.n_long[0], 1u)] = (uint32_t)row;
+            else if (ee - eb >= TR_LONG) a.long_rows[a.n_rows - 1 - atomicAdd(&a.n_long[1], 1u)] = (uint32_t)row;
+        }
     }
 }
 
@@ -971,8 +980,8 @@ __global__ __launch_bounds__(TC_ROWS * WAVE) void k_tile_counts(TileArgs a) {
 // while this one is added, and the carry moves by DPP instead of eight LDS
 // permutes.
 // Measured against the 32-run kernel with maps: 120 -> 43 us on a line of 61
-// glyphs, 422 -> 203 us on 10,000 glyphs (81% of the SIMDs' VALU cycles), 2,684 ->
-// 930 us on 24 star blobs of 1,000-20,000 cubics.
+// glyphs, 422 -> 180 us on 10,000 glyphs (VALU-bound), 2,684 ->
+// 560 us on 24 star blobs of 1,000-20,000 cubics.
 constexpr int TR_SLOTS = 15;  // increments per run
 constexpr int TR_BLOCK = WAVE;  // runs replayed per block
 
@@ -997,36 +1006,39 @@ static inline uint32_t row_grid(int64_t rows, int64_t cap) {
 
 // The increments of a run from the DDA state at its first one (p0: that
 // increment's start point) into their slots from inc[0] on, `dir` apart, and the
-// run's bit into the hit words of its pixels; CARRY: every active lane's line is finite, so each
-// increment's start point is the previous one's end point (see
-// dda_increment_carried).
-template <bool CARRY>
+// run's bit into the hit words of its pixels.  FAST: every active lane's line is
+// one that FastWalk covers.  The pixel within the tile is two nibbles (y above x);
+// leaving 0..7 on either axis sets a nibble's top bit.
+template <bool FAST>
 __device__ inline void tr_replay_steps(float2* inc, int dir, uint32_t* hit, uint32_t bit, Dda& d, V2 p0, bool finite,
                                        Counters* cnt) {
-    uint32_t lx = (uint32_t)(d.x & 7), ly = (uint32_t)(d.y & 7);
-    const uint32_t lxd = (uint32_t)(int32_t)d.x_dir, lyd = (uint32_t)(int32_t)d.y_dir;
+    uint32_t at = (uint32_t)(((d.y & 7) << 4) | (d.x & 7));
+    const uint32_t xd = (uint32_t)(int32_t)d.x_dir, yd = (uint32_t)((int32_t)d.y_dir * 16);
+    auto put = [&](float area, float height) {
+        *inc = make_float2(area, height);
+        inc += dir;
+        atomicOr(&hit[at - ((at >> 4) << 3)], bit);
+    };
+    if constexpr (FAST) {
+        FastWalk w;
+        w.init(d, p0);
+        for (;;) {  // (at most 15 steps: each moves one pixel on, the same way along its axis)
+            float area, height;
+            bool y;
+            const bool end = w.step(area, height, y);
+            put(area, height);
+            at += y ? yd : xd;
+            if (end || (at & 0x88u)) break;
+        }
+        return;
+    }
     bool ended = false;
     for (int k = 0; k < TR_SLOTS; k++) {
         float area, height;
-        dda_increment_carried(d, p0, CARRY || finite, area, height);
-        *inc = make_float2(area, height);
-        inc += dir;
-        atomicOr(&hit[(ly << 3) | lx], bit);
-        // dda_step, with the in-tile pixel moved alongside
-        float c;
-        if (d.row_t1 < d.col_t1) {
-            c = d.row_t1;
-            d.row_t1 = fminf(d.row_t1 + d.y_step, 1.0f);
-            d.y = wrap16(d.y + d.y_dir);
-            ly += lyd;
-        } else {
-            c = d.col_t1;
-            d.col_t1 = fminf(d.col_t1 + d.x_step, 1.0f);
-            d.x = wrap16(d.x + d.x_dir);
-            lx += lxd;
-        }
-        d.t0 = c;
-        if (c == 1.0f || (lx | ly) > 7u) {
+        dda_increment_carried(d, p0, finite, area, height);
+        put(area, height);
+        at += d.row_t1 < d.col_t1 ? yd : xd;
+        if (dda_step(d) || (at & 0x88u)) {
             ended = true;
             break;
         }
@@ -1034,27 +1046,50 @@ __device__ inline void tr_replay_steps(float2* inc, int dir, uint32_t* hit, uint
     if (!ended) atomicOr(&cnt->error, (uint32_t)ERR_REPLAY);
 }
 
+// A wave's LDS accesses before and after this point stay in their order (they
+// are executed in order; this holds the compiler to it).
+__device__ inline void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 template <int CTRL>
 __device__ inline float dpp_f(float old, float v) {
     return __uint_as_float(dpp<CTRL>(__float_as_uint(old), __float_as_uint(v)));
 }
 
-__global__ __launch_bounds__(WAVE) void k_tile_rows(TileArgs a) {
-    __shared__ float2 inc[TR_BLOCK * TR_SLOTS];
-    __shared__ uint32_t hit[2][64];  // pixel p, bit j: run 32 w + j visits p
-    const int lane = threadIdx.x;
+// PAIRED: the long rows, two waves each, a block apart: one replays block i while
+// the other adds block i - 1 and writes its tiles, one barrier per block.  Rows vary
+// (24 blobs: 1,480 runs on average, 11,900 at most), a row's blocks run one after
+// another, and a wave alone on its SIMD issues an instruction only every 9 cycles:
+// with a wave per row the longest row took as long as the whole kernel, at 1.6
+// waves per SIMD on average.  The longest of them start first.  The other rows, a
+// wave each, run in a launch beside it.
+struct TrBuf {
+    float2 inc[TR_BLOCK * TR_SLOTS];
+    uint32_t hit[2][64];       // pixel p, bit j: run 32 w + j visits p
+    unsigned long long alike;  // the runs whose slots are x + y
+};
+
+template <bool PAIRED>
+__global__ __launch_bounds__(PAIRED ? 2 * WAVE : WAVE) void k_tile_rows(TileArgs a, uint32_t n_longest) {
+    __shared__ TrBuf buf[PAIRED ? 2 : 1];
+    const int lane = threadIdx.x & (WAVE - 1);
     // Lane -> pixel: 16 lanes hold two pixel rows interleaved, so that a move of
     // two lanes is the next pixel of the same row and the first two lanes, which
     // have no source, keep the carry.
     const uint32_t px = (uint32_t)(lane >> 1) & 7u, py = (uint32_t)((lane >> 4) << 1) | (uint32_t)(lane & 1);
     const uint32_t pix = (py << 3) | px, slot_alike = px + py, slot_unlike = px + 7u - py;
     const uint32_t xmask = (1u << a.xbits) - 1;
-    for (int64_t row = xcd_first_row(); row < a.n_rows; row += gridDim.x) {
+    const bool replays = !PAIRED || threadIdx.x < WAVE, adds = !PAIRED || threadIdx.x >= WAVE;
+    int64_t row = xcd_first_row();
+    if (PAIRED) row = a.long_rows[blockIdx.x < n_longest ? blockIdx.x : a.n_rows - 1 - (blockIdx.x - n_longest)];
+    for (; row < a.n_rows; row += PAIRED ? a.n_rows : (int64_t)gridDim.x) {
         const PathGrid G = a.grid[a.row_path[row]];
         if (row - (int64_t)G.row_base >= G.h) continue;  // the empty-path row (k_path_out)
         const uint32_t eb = __builtin_amdgcn_readfirstlane(a.row_begin[row]);
         const uint32_t ee = __builtin_amdgcn_readfirstlane(a.row_end[row]);
-        if (ee <= eb) continue;
+        if (ee <= eb || (ee - eb >= TR_LONG) != PAIRED) continue;
         const int32_t ty = G.ty0 + (int32_t)(row - (int64_t)G.row_base);
         const uint64_t off = a.row_off[row];
         const uint32_t row_tiles = (uint32_t)(off >> 32), row_spans = (uint32_t)off;
@@ -1064,7 +1099,8 @@ __global__ __launch_bounds__(WAVE) void k_tile_rows(TileArgs a) {
         uint32_t nt = 0, ns = 0;
         float pa = 0.0f, ph = 0.0f;  // this pixel's sums of the open tile
         uint32_t h0 = 0, h1 = 0;     // this pixel's hit words of the block
-        uint64_t alike = 0;          // the block's runs whose slots are x + y
+        uint64_t alike = 0;
+        const float2* inc = nullptr;
         // two hits at a time: their reads are in flight together
         auto add_runs = [&](uint32_t h, uint32_t al, uint32_t lo, uint32_t hi, const float2* incs) {
             uint32_t m = h & (0xffffffffu << lo) & (0xffffffffu >> (32u - hi));
@@ -1100,6 +1136,14 @@ __global__ __launch_bounds__(WAVE) void k_tile_rows(TileArgs a) {
             }
             ns++;
         };
+        int32_t txy = 0;
+        auto store_xy = [&](uint32_t n) {  // of the last n tiles
+            if ((uint32_t)lane < n) {
+                int16_t* xy = a.tile_xy + 2 * (size_t)(row_tiles + nt - n + (uint32_t)lane);
+                xy[0] = (int16_t)txy;
+                xy[1] = (int16_t)(ty * TILE);
+            }
+        };
         auto tile = [&](int32_t x) {
             // (d)(e) the fold along each pixel row: after k moves the lanes of
             // pixels 0..k hold ((carry + h0) + h1) ..., the later ones not yet
@@ -1116,11 +1160,10 @@ __global__ __launch_bounds__(WAVE) void k_tile_rows(TileArgs a) {
             a.tile_alpha[(size_t)ti * 64 + pix] = (uint8_t)(uint32_t)fminf(cov * 256.0f, 255.0f);
             pa = 0.0f;
             ph = 0.0f;
-            if (lane == 0) {
-                a.tile_xy[2 * ti] = (int16_t)((G.tx0 + x) * TILE);
-                a.tile_xy[2 * ti + 1] = (int16_t)(ty * TILE);
-            }
+            // the tiles' coordinates wait in lanes, stored 64 at a time
+            if (lane == (int)(nt & (WAVE - 1))) txy = (G.tx0 + x) * TILE;
             nt++;
+            if ((nt & (WAVE - 1)) == 0) store_xy(WAVE);
         };
         // the entries of a block, their records and lines
         auto load = [&](const uint32_t* p, uint32_t b, uint32_t none) {
@@ -1138,59 +1181,89 @@ __global__ __launch_bounds__(WAVE) void k_tile_rows(TileArgs a) {
         uint32_t k1 = load(a.keys, eb, 0u), v1 = load(a.vals, eb, 0x80000000u);
         uint32_t k2 = load(a.keys, eb + TR_BLOCK, 0u), v2 = load(a.vals, eb + TR_BLOCK, 0x80000000u);
         uint32_t k3 = load(a.keys, eb + 2 * TR_BLOCK, 0u), v3 = load(a.vals, eb + 2 * TR_BLOCK, 0x80000000u);
-        RunRec r1 = load_rec(v1), r2 = load_rec(v2);
-        float4 l1 = load_line(v1, r1);
-        for (uint32_t b = eb; b < ee; b += TR_BLOCK) {
-            // (c) replay the block's entries, one run per lane
-            const uint32_t key = k1, v = v1;
-            const RunRec r = r1;
-            const float4 L = l1;
+        RunRec r1{}, r2{};
+        float4 l1{};
+        if (replays) {
+            r1 = load_rec(v1);
+            r2 = load_rec(v2);
+            l1 = load_line(v1, r1);
+        }
+        uint32_t key = 0, v = 0, key0 = 0, v0 = 0;  // of the block replayed, and of the one before
+        const uint32_t n_blk = (ee - eb + TR_BLOCK - 1) / TR_BLOCK;
+        for (uint32_t i = 0; i < n_blk + (PAIRED ? 1u : 0u); i++) {
+            const uint32_t b = eb + i * TR_BLOCK;
+            key0 = key;
+            v0 = v;
+            key = k1;
+            v = v1;
             k1 = k2;
             v1 = v2;
-            r1 = r2;
-            l1 = load_line(v1, r1);
             k2 = k3;
             v2 = v3;
-            r2 = load_rec(v2);
             k3 = load(a.keys, b + 3 * TR_BLOCK, 0u);
             v3 = load(a.vals, b + 3 * TR_BLOCK, 0x80000000u);
-            __syncthreads();  // the previous block's increments are read
-            hit[0][lane] = 0;
-            hit[1][lane] = 0;
-            __syncthreads();
-            bool al = false;
-            if (!(v >> 31)) {
-                Dda d;
-                const V2 last = mk(L.x, L.y), point = mk(L.z, L.w);
-                if (r.line >> 31) {
-                    dda_init(d, last, point);
-                } else {
-                    dda_consts(d, last, point);
-                    d.x = (int16_t)(r.xy & 0xffffu);
-                    d.y = (int16_t)(r.xy >> 16);
-                    d.row_t1 = r.row_t1;
-                    d.col_t1 = r.col_t1;
-                    d.t0 = 0.0f;
-                    dda_step(d);
+            if (replays && i < n_blk) {
+                // (c) replay the block's entries, one run per lane
+                TrBuf& B = buf[PAIRED ? i & 1u : 0u];
+                const RunRec r = r1;
+                const float4 L = l1;
+                r1 = r2;
+                l1 = load_line(v1, r1);
+                r2 = load_rec(v2);
+                B.hit[0][lane] = 0;
+                B.hit[1][lane] = 0;
+                wave_lds_order();
+                bool al = false;
+                if (!(v >> 31)) {
+                    Dda d;
+                    const V2 last = mk(L.x, L.y), point = mk(L.z, L.w);
+                    if (r.line >> 31) {
+                        dda_init(d, last, point);
+                    } else {
+                        dda_consts(d, last, point);
+                        d.x = (int16_t)(r.xy & 0xffffu);
+                        d.y = (int16_t)(r.xy >> 16);
+                        d.row_t1 = r.row_t1;
+                        d.col_t1 = r.col_t1;
+                        d.t0 = 0.0f;
+                        dda_step(d);
+                    }
+                    const bool finite = line_finite(last, point);
+                    const V2 p0 = dda_point(d, d.t0);
+                    // (a direction is 0 only where a coordinate is not finite: that axis takes no step)
+                    al = d.x_dir == d.y_dir || d.x_dir == 0 || d.y_dir == 0;
+                    const int dir = d.x_dir ? d.x_dir : d.y_dir;
+                    float2* out = B.inc + lane * TR_SLOTS + (al ? (d.x & 7) + (d.y & 7) : (d.x & 7) + 7 - (d.y & 7));
+                    uint32_t* hw = B.hit[lane >> 5];
+                    const uint32_t bit = 1u << (lane & 31);
+                    if (__ballot(!fast_walk_ok(last, point)) == 0) tr_replay_steps<true>(out, dir, hw, bit, d, p0, finite, a.cnt);
+                    else tr_replay_steps<false>(out, dir, hw, bit, d, p0, finite, a.cnt);
                 }
-                const bool finite = line_finite(last, point);
-                const V2 p0 = dda_point(d, d.t0);
-                // (a direction is 0 only where a coordinate is not finite: that axis takes no step)
-                al = d.x_dir == d.y_dir || d.x_dir == 0 || d.y_dir == 0;
-                const int dir = d.x_dir ? d.x_dir : d.y_dir;
-                float2* out = inc + lane * TR_SLOTS + (al ? (d.x & 7) + (d.y & 7) : (d.x & 7) + 7 - (d.y & 7));
-                uint32_t* hw = hit[lane >> 5];
-                const uint32_t bit = 1u << (lane & 31);
-                if (__ballot(!finite) == 0) tr_replay_steps<true>(out, dir, hw, bit, d, p0, finite, a.cnt);
-                else tr_replay_steps<false>(out, dir, hw, bit, d, p0, finite, a.cnt);
+                alike = __ballot(al);
+                if (PAIRED && lane == 0) B.alike = alike;
+                wave_lds_order();
             }
-            __syncthreads();
-            h0 = hit[0][pix];
-            h1 = hit[1][pix];
-            alike = __ballot(al);
-            bins.step(key, v, min((uint32_t)TR_BLOCK, ee - b), xmask, part, tile, span);
+            if (adds && (!PAIRED || i > 0)) {
+                const TrBuf& B = buf[PAIRED ? (i - 1u) & 1u : 0u];
+                inc = B.inc;
+                h0 = B.hit[0][pix];
+                h1 = B.hit[1][pix];
+                if (PAIRED) {
+                    const unsigned long long w = B.alike;
+                    alike = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(w >> 32)) << 32) |
+                            (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)w);
+                }
+                const uint32_t b0 = PAIRED ? b - TR_BLOCK : b;
+                bins.step(PAIRED ? key0 : key, PAIRED ? v0 : v, min((uint32_t)TR_BLOCK, ee - b0), xmask, part, tile,
+                          span);
+                wave_lds_order();
+            }
+            if (PAIRED) __syncthreads();
         }
-        bins.close(tile, span);
+        if (adds) {
+            bins.close(tile, span);
+            store_xy(nt & (WAVE - 1));
+        }
     }
 }
 
@@ -1800,8 +1873,9 @@ struct HostTotals {
     uint32_t max_w;
     uint32_t rows;
     uint64_t dda;     // (runs << 32) | entries
-    uint32_t groups;
+    uint32_t windows;  // of the unordered tile stage
     uint32_t pad;
+    uint32_t n_long[2];  // long rows of the ordered one (TileArgs::n_long); read with out
     uint64_t out;     // (tiles << 32) | spans
     uint64_t entries;
 };
@@ -1840,7 +1914,7 @@ static int run_plain_pass(Context* ctx, const SegInput& in, OutputDesc& out, hip
     HIPCHK(ctx->totals.ensure(256));
     if (!ctx->host_pinned) HIPCHK(hipHostMalloc(&ctx->host_pinned, 4096));
     Counters* cnt = ctx->counters.as<Counters>();
-    uint64_t* tot = ctx->totals.as<uint64_t>();  // [0] lines, [1] rows, [2] dda, [3] groups, [4] out
+    uint64_t* tot = ctx->totals.as<uint64_t>();  // [0] lines, [1] rows, [2] dda, [3] long rows, [4] out, [6] windows
     HostTotals* ht = reinterpret_cast<HostTotals*>(ctx->host_pinned);
     fill<uint32_t>(reinterpret_cast<uint32_t*>(cnt), 64, 0u, s);
     fill<uint64_t>(tot, 32, 0ull, s);
@@ -1983,9 +2057,9 @@ static int run_plain_pass(Context* ctx, const SegInput& in, OutputDesc& out, hip
         hipLaunchKernelGGL(k_rows_setup, dim3(grid_for(NP, PR_WAVES)), dim3(PR_WAVES * WAVE), 0, s, grid, NP, pwbase,
                            ctx->row_path.as<uint32_t>(), rwbase);
         HIPCHK(hipGetLastError());
-        HIPCHK(hipMemcpyAsync(&ht->groups, nb_dev, 4, hipMemcpyDeviceToHost, s));
+        HIPCHK(hipMemcpyAsync(&ht->windows, nb_dev, 4, hipMemcpyDeviceToHost, s));
         HIPCHK(hipStreamSynchronize(s));
-        const int64_t NB = ht->groups;
+        const int64_t NB = ht->windows;
         HIPCHK(ctx->u_bcnt.ensure((size_t)std::max<int64_t>(NB, 1) * 4));
         HIPCHK(ctx->u_bbeg.ensure((size_t)(NB + 1) * 4));
         HIPCHK(ctx->u_bcur.ensure((size_t)std::max<int64_t>(NB, 1) * 4));
@@ -2137,12 +2211,15 @@ static int run_plain_pass(Context* ctx, const SegInput& in, OutputDesc& out, hip
     ta.span_xy = out.span_xy;
     ta.span_w = out.span_w;
     ta.cnt = cnt;
+    HIPCHK(ctx->long_rows.ensure(ROWS * 4));
+    ta.long_rows = ctx->long_rows.as<uint32_t>();
+    ta.n_long = reinterpret_cast<uint32_t*>(&tot[3]);
     const uint32_t tile_blocks = (uint32_t)std::min<int64_t>((ROWS + TC_ROWS - 1) / TC_ROWS, 1 << 20);
     hipLaunchKernelGGL(k_tile_counts, dim3(tile_blocks), dim3(TC_ROWS * WAVE), 0, s, ta);
     HIPCHK(launch_scan<uint64_t>(ctx, ROWS, LoadU64{ta.row_cnt}, StoreU64{ctx->row_off.as<uint64_t>()}, OpAdd(),
                                  0ull, &tot[4], s));
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(&ht->out, &tot[4], 8, hipMemcpyDeviceToHost, s));
+    HIPCHK(hipMemcpyAsync(ht->n_long, &tot[3], 16, hipMemcpyDeviceToHost, s));  // and out
     HIPCHK(hipMemcpyAsync(&ht->error, &cnt->error, 4, hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
     if (ht->error & (ERR_BBOX | ERR_REPLAY)) return -3;
@@ -2158,7 +2235,25 @@ static int run_plain_pass(Context* ctx, const SegInput& in, OutputDesc& out, hip
         if (!ctx->ev[1]) HIPCHK(hipEventCreate(&ctx->ev[1]));
         HIPCHK(hipEventRecord(ctx->ev[0], s));
     }
-    hipLaunchKernelGGL(k_tile_rows, dim3(row_grid(ROWS, 1 << 20)), dim3(WAVE), 0, s, ta);
+    const uint32_t n_long = ht->n_long[0] + ht->n_long[1];
+    if (n_long) {
+        // beside each other: the long rows alone leave the chip half empty
+        if (!ctx->own_stream) HIPCHK(hipStreamCreateWithFlags(&ctx->own_stream, hipStreamNonBlocking));
+        for (auto& e : ctx->side_ev)
+            if (!e) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        HIPCHK(hipEventRecord(ctx->side_ev[0], s));
+        HIPCHK(hipStreamWaitEvent(ctx->own_stream, ctx->side_ev[0], 0));
+        hipLaunchKernelGGL(k_tile_rows<true>, dim3(n_long), dim3(2 * WAVE), 0, ctx->own_stream, ta, ht->n_long[0]);
+    }
+    hipLaunchKernelGGL(k_tile_rows<false>, dim3(row_grid(ROWS, 1 << 20)), dim3(WAVE), 0, s, ta, 0u);
+    if (n_long) {
+        hipError_t e = hipEventRecord(ctx->side_ev[1], ctx->own_stream);
+        if (e == hipSuccess) e = hipStreamWaitEvent(s, ctx->side_ev[1], 0);
+        if (e != hipSuccess) {  // nothing of the call runs on after it
+            (void)hipStreamSynchronize(ctx->own_stream);
+            return map_hip_error(e);
+        }
+    }
     if (ctx->timing) HIPCHK(hipEventRecord(ctx->ev[1], s));
     hipLaunchKernelGGL(k_path_out, dim3(grid_for(NP, 256)), dim3(256), 0, s, grid, NP, ta.row_off,
                        (const uint64_t*)&tot[4], out.path_tile_start, out.path_tile_count, out.path_span_start,

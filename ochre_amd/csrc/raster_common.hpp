@@ -235,6 +235,55 @@ __device__ inline void walk_line(V2 last, V2 point, Sink& sink) {
 }
 
 
+// The DDA at one pixel after another (dda_increment_carried, then dda_step) for
+// lines with finite coordinates within +-HUGE_COORD, in about 25 operations a step
+// where the general form takes 45 and two divergent branches: no coordinate wraps
+// or is NaN, so the smaller crossing parameter is a select by the comparison that
+// the step needs anyway, both axes share one addition and clamp, and the pixel's
+// right edge is kept as a float.  The same f32 operations on the same values (up to
+// the sign of a zero parameter, which no sum sees).
+struct FastWalk {
+    float ax, ay, bx, by;  // the line
+    float xs, ys, sx;      // parameter steps, and the direction along x
+    float row, col;        // next crossing parameters
+    float right;           // right edge of the pixel
+    float p0x, p0y;        // start point of its increment
+    __device__ void init(const Dda& d, V2 p0) {
+        ax = d.last.x;
+        ay = d.last.y;
+        bx = d.point.x;
+        by = d.point.y;
+        xs = d.x_step;
+        ys = d.y_step;
+        sx = (float)d.x_dir;
+        row = d.row_t1;
+        col = d.col_t1;
+        right = (float)(d.x + 1);
+        p0x = p0.x;
+        p0y = p0.y;
+    }
+    // The increment at the current pixel, then a step: y says along which axis.
+    // Returns true when the line has ended.
+    __device__ bool step(float& area, float& height, bool& y) {
+        y = row < col;
+        const float t = y ? row : col, u = 1.0f - t;
+        const float p1x = u * ax + t * bx, p1y = u * ay + t * by;
+        height = p1y - p0y;
+        area = 0.5f * height * ((right - p0x) + (right - p1x));
+        p0x = p1x;
+        p0y = p1y;
+        const float n = fminf(t + (y ? ys : xs), 1.0f);
+        row = y ? n : row;
+        col = y ? col : n;
+        right += y ? 0.0f : sx;
+        return t == 1.0f;
+    }
+};
+// Lines that FastWalk covers.
+__device__ inline bool fast_walk_ok(V2 a, V2 b) {
+    return fabsf(a.x) <= HUGE_COORD && fabsf(a.y) <= HUGE_COORD && fabsf(b.x) <= HUGE_COORD && fabsf(b.y) <= HUGE_COORD;
+}
+
 // Lines that line_counts and line_tiles cover: finite, within +-30000, at
 // most 4096 px per axis (no i16 wrap, far below the walk's step limit).
 __device__ inline bool chain_walk_ok(V2 last, V2 point) {

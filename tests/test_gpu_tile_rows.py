@@ -30,3 +30,13 @@ def test_rows_of_runs_around_a_block(gpu_ctx, n, tiles, rows):
     b = W.from_paths(paths, np.array([[1, 0, 0, 1, 0, 0], [1, 0, 0, 1, -13.5, 4.25], [1, 0, 0, 1, 7.0, -9.0]], np.float32))
     stats = compare(oracle_ref.run_batch(b), run_to_host(gpu_ctx, b, "plain"), max_lsb=0)
     assert stats["bit_exact_fraction"] == 1.0
+
+
+@pytest.mark.parametrize("n,tiles", [(2040, 1), (2047, 1), (2048, 1), (2049, 1), (2111, 3), (6143, 1), (6145, 2), (1500, 30)])
+def test_rows_of_two_waves(gpu_ctx, n, tiles):
+    """Rows of 2,048 entries and more (two waves to a row) beside shorter ones."""
+    from ochre_amd.device import run_to_host
+    paths = [_zigzag(n, tiles, 1, n), _zigzag(90, 5, 2, 1), _zigzag(n + 64, tiles, 2, 3)]
+    b = W.from_paths(paths, W.IDENTITY)
+    stats = compare(oracle_ref.run_batch(b), run_to_host(gpu_ctx, b, "plain"), max_lsb=0)
+    assert stats["bit_exact_fraction"] == 1.0
