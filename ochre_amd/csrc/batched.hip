@@ -542,11 +542,14 @@ __device__ void fused_path(const FusedIn& in, const FusedOut& out, FusedCtl* ctl
             }
         }
     }
+    if (ADJ) {
+        // (the adjoint takes its coverage from the f64 geometry: emitting and
+        // committing the f32 increments in front of it was half of its walks,
+        // 1,447 -> 1,137 us on 4,096 paths of 16 cubics)
+        adjoint_backward<TC>(in, adj, ctl, sc, asc, s, p, L, NT, NS, tx0, ty0, GW, GH);
+        return;
+    }
     if (NT == 0) {  // no increments: one all-zero tile at (0, 0) (rasterizer.rs:193-198)
-        if (ADJ) {
-            adjoint_backward<TC>(in, adj, ctl, sc, asc, s, p, L, 0, NS, tx0, ty0, GW, GH);
-            return;
-        }
         if (lane < 4) reinterpret_cast<uint4*>(out.tile_alpha + tb * 64)[lane] = make_uint4(0, 0, 0, 0);
         if (out.tile_cov)
             for (int k = lane; k < 64; k += WAVE) out.tile_cov[tb * 64 + k] = 0.0f;
@@ -697,25 +700,8 @@ __device__ void fused_path(const FusedIn& in, const FusedOut& out, FusedCtl* ctl
             }
         }
         __syncthreads();
-        if (ADJ) {
-            // keep v = accum + area of every pixel (rank order) for the loss
-            if ((uint32_t)lane < nt) {
-                const int t = lane;
-                float* tv = reinterpret_cast<float*>(asc + A_OFF_TILES) + (size_t)(r0 + t) * 128;
-#pragma unroll
-                for (int y = 0; y < 8; y++) {
-                    float accum = s.u.a.cin[t * 8 + y];
-#pragma unroll
-                    for (int x = 0; x < 8; x++) {
-                        const int k = t * F_TSTRIDE + y * 8 + x;
-                        tv[y * 8 + x] = accum + s.u.a.acc_a[k];
-                        accum += s.u.a.acc_h[k];
-                    }
-                }
-            }
-        }
         // quantise and store (rasterizer.rs:231-241)
-        if (!ADJ && (uint32_t)lane < nt) {
+        if ((uint32_t)lane < nt) {
             const int t = lane;
             const int ty = (int)(s.chunk_tile[t] >> 8), tx = (int)(s.chunk_tile[t] & 0xffu);
             uint32_t words[16];
@@ -748,7 +734,6 @@ __device__ void fused_path(const FusedIn& in, const FusedOut& out, FusedCtl* ctl
         }
         __syncthreads();
     }
-    if (ADJ) adjoint_backward<TC>(in, adj, ctl, sc, asc, s, p, L, NT, NS, tx0, ty0, GW, GH);
 }
 
 template <int TC>
