@@ -361,7 +361,7 @@ def time_modes(ctx, batch, db, out, modes, steps, warmup, keep_outputs):
             ctx.set_timing(True)
             time_steps(fn, steps, 1)
             kernels = {}
-            for k in ("k_dense", "k_fused", "k_row_tiles", "k_tile_rows"):
+            for k in ("k_dense", "k_row_tiles", "k_tile_rows"):
                 t, n = ctx.timing(k)
                 if n:
                     kernels[k] = t / n  # the last two: the plain pipeline over the handed-on paths
@@ -376,7 +376,7 @@ def time_modes(ctx, batch, db, out, modes, steps, warmup, keep_outputs):
             ctx.set_timing(False)
             set_batched_params(ctx, bp["waves_per_cu"], bp["paths_per_pop"], bp["tiles_per_chunk"],
                                graph=bool(bp["graph"]))
-            kname = "k_dense" if bp.get("dense") else "k_fused"
+            kname = "k_dense" if bp.get("dense") else "k_tile_rows"
             if kernels.get("k_row_tiles", 0.0) > kernels.get(kname, 0.0):
                 kname = "k_row_tiles"
         torch.cuda.synchronize()

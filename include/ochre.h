@@ -174,12 +174,13 @@ void ochre_context_destroy(ochre_context* ctx);
 int ochre_rasterize_plain(ochre_context* ctx, const ochre_path_batch* in, ochre_batch_output* out,
                           void* stream);
 
-/* The batched pipeline: one persistent work-queue launch (one wave64 per
- * path; the launch and its queue reset are replayed from a captured HIP
- * graph), for batches of many small paths.  Paths whose tile grid exceeds
- * 32 x 32 tiles or which flatten to more than 8192 lines are handed to the
- * plain pipeline within the same call.  Tiles of a path are contiguous and in
- * row-major order, but paths are laid out in the order they finish. */
+/* The batched pipeline: the dense kernels, persistent over a device queue of
+ * paths (a workgroup per path; the launches and their queue reset may be
+ * replayed from a captured HIP graph), for batches of many small paths.  Paths
+ * over the largest dense instance go to the plain pipeline's unordered tile
+ * stage within the same call; with the dense kernels off every path takes the
+ * plain pipeline, in passes of bounded scratch.  Tiles of a path are contiguous
+ * and in row-major order, but paths are laid out in the order they finish. */
 int ochre_rasterize_batched(ochre_context* ctx, const ochre_path_batch* in, ochre_batch_output* out,
                             void* stream);
 
@@ -237,21 +238,20 @@ int ochre_build_atlas(ochre_context* ctx, const ochre_batch_output* in, int64_t 
                       uint32_t* indices, int64_t index_capacity, int64_t* n_vertices, int64_t* n_indices,
                       void* stream);
 
-/* Tunables of the batched pipeline (the autotuner sets them): persistent
- * waves per compute unit (1-32), paths taken per queue pop (1-1024), tiles
- * accumulated per pass in LDS (16 or 32: fewer tiles, more waves per CU),
- * and whether to replay the launch from a HIP graph. */
+/* Settings of the batched pipeline: waves_per_cu (1-32), paths_per_pop (1-1024)
+ * and tiles_per_chunk (16 or 32) are kept and reported, and choose nothing since
+ * the ordered path of the call is the plain pipeline; use_graph: replay the
+ * dense launches from a HIP graph. */
 int ochre_context_set_batched_params(ochre_context* ctx, int waves_per_cu, int paths_per_pop, int tiles_per_chunk,
                                      int use_graph);
 int ochre_context_get_batched_params(ochre_context* ctx, int* waves_per_cu, int* paths_per_pop, int* tiles_per_chunk,
                                      int* use_graph);
 
-/* The dense single-walk kernel (on by default) runs in front of the ordered
- * one and takes every path whose tile grid (line bounding box + a 2 px
+/* The dense single-walk kernel (on by default) takes every path whose tile grid (line bounding box + a 2 px
  * margin) has at most 64 tiles: one DDA walk adds each increment to its
  * pixel's sums with LDS float atomics, so f32 sums are taken in arrival
  * order and an alpha can differ from the ordered result by 1 LSB (tile and
- * span sets are exact).  Off: every path goes through the ordered kernel,
+ * span sets are exact).  Off: every path goes through the plain pipeline,
  * whose sums follow emission order.  groups_per_cu 1-8 resident workgroups,
  * waves_per_group 2, 4 or 8 (waves sharing one path; with 8, at most 2
  * workgroups per CU are resident). */
@@ -264,9 +264,9 @@ int ochre_context_get_dense_params(ochre_context* ctx, int* enabled, int* groups
  * faster; the autotuner tries both). */
 int ochre_context_set_dense_small(ochre_context* ctx, int groups_per_cu);
 int ochre_context_get_dense_small(ochre_context* ctx, int* groups_per_cu);
-/* A 256-tile dense instance (one workgroup of 16 waves and 130 KB of LDS per
+/* A 256-tile dense instance (one workgroup of 8 waves and 140 KB of LDS per
  * CU) behind the 64-tile one, over the paths it hands on (grids of 65-256
- * tiles go there instead of to the ordered kernel); enabled 0 or 1, default
+ * tiles go there instead of to the plain pipeline); enabled 0 or 1, default
  * 1.  The autotuner tries both. */
 int ochre_context_set_dense_large(ochre_context* ctx, int enabled);
 int ochre_context_get_dense_large(ochre_context* ctx, int* enabled);
@@ -311,10 +311,8 @@ int ochre_coverage_adjoint(ochre_context* ctx, const ochre_path_batch* in, const
 /* Autotuner: with the dense kernel on, times every (workgroups per CU
  * {1,2,3,4}, waves per workgroup {2,4,8}) of the 64-tile dense launch, then
  * the small-grid instance {off, 4, 6, 8 workgroups per CU}, the 256-tile
- * instance {off, on}, then waves per CU {1,2,4,8} of the ordered kernel
- * behind them; with it off,
- * every combination of waves per CU {2,3,4,6,8,12}, paths per pop {1,2,4,8}
- * and tiles per chunk {16,32} of the ordered launch.  Each configuration is
+ * instance {off, on}; with it off the call has no launch shape, and is timed
+ * once.  Each configuration is
  * timed on the caller's batch (`reps` calls, median); the fastest is kept in
  * the context and every measurement reported in `results` (up to
  * max_results entries). */

@@ -1,26 +1,14 @@
-// Batched pipeline: one persistent launch works through a queue of paths,
-// one wave64 per path, everything for a path on one CU:
-//   flatten   lane per command (64 at a time, wave scans carry the point /
-//             conic / last-Move state), lines to per-wave scratch
-//   count     lane per line, lanes refilled from the line list as they finish
-//             (no lane idles while one long line is walked); marks occupied
-//             tiles and sums tile-row crossings in LDS
-//   allocate  tile and span counts -> one atomic per path for its output
-//             range; spans written directly (integer winding)
-//   emit      lane per line again, each increment (pixel, area, height)
-//             written to scratch at its emission index
-//   commit    64 increments at a time in emission order into LDS tile
-//             accumulators; lanes hitting the same pixel are found by ballot
-//             matching and commit in lane order, so every pixel's f32 sum is
-//             taken in the reference's emission order (rasterizer.rs:221-228)
-//   finalize  row carry (rasterizer.rs:233-250) and quantisation, 64 B stores
-// Paths too large for a wave (grid > 32x32 tiles or > 8192 lines) are
-// deferred to the plain pipeline by the host driver.
+// Batched pipeline: the dense kernels (dense.inc), persistent over a device queue
+// of paths, then the plain pipeline's unordered tile stage over the paths that no
+// dense instance holds.  With the dense kernels off the call is the plain pipeline
+// itself, whose sums follow emission order.  (A one-wave-per-path ordered kernel
+// that took these paths before, flattening, counting, emitting and committing a
+// path's increments on one wave, is slower at every size measured: 61 glyphs of
+// 12-48 px 666 us against 300, 10,000 of them 1,621 against 880, 300 of 12-120 px
+// 4,174 against 387, one of 250 px 7,373 against 276.)
 //
-// With the dense mode on (the default), k_dense (dense.inc) runs first and
-// takes every path whose tile grid fits its LDS grid in a single walk with
-// order-independent accumulation; k_fused then works through the paths it
-// handed on.
+// Also here: the coverage adjoint (adjoint.inc, adjoint_large.inc), the single
+// fill (single.inc) and the allocation-free dense chain.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -35,10 +23,9 @@
 namespace ochre {
 
 constexpr int F_LCAP = 8192;   // lines per path
-constexpr int F_ICAP = 8192;   // increments per commit batch
 constexpr int F_GRID = 32;     // tile grid side (256 px)
 constexpr int F_TSTRIDE = 65;  // accumulator stride per tile (bank spread)
-constexpr size_t F_SCRATCH = (size_t)F_LCAP * 16 + (size_t)(F_LCAP + 1) * 4 + 12 + (size_t)F_ICAP * 16;
+constexpr size_t F_SCRATCH = (size_t)F_LCAP * 32;  // per wave of the adjoint: its path's lines and their gradients
 constexpr uint32_t F_INVALID = 0xffffffffu;
 
 struct FusedIn {
@@ -55,13 +42,7 @@ struct FusedIn {
     // k_dense) instead of 0 .. n_paths
     const uint32_t* ids = nullptr;
     const uint32_t* n_ids = nullptr;
-    // more handed-on paths than this go to the plain pipeline whole: one wave
-    // per path is slow on the large paths the dense kernels hand on, and the
-    // plain pipeline's fixed cost is repaid from a few hundred of them
-    uint32_t defer_above = 0xffffffffu;
 };
-
-constexpr uint32_t F_DEFER_ABOVE = 512;  // handed-on paths beyond which k_fused defers them all
 
 struct FusedOut {
     int16_t* tile_xy;
@@ -79,17 +60,16 @@ struct FusedOut {
 
 struct FusedCtl {
     uint32_t queue;     // path queue of the first kernel of the launch
-    uint32_t deferred;  // paths handed to the plain pipeline
+    uint32_t deferred;  // paths over the kernel's limits (the adjoint, the single fill)
     uint32_t error;
     uint32_t dq;        // paths handed on by k_dense
     unsigned long long tiles;
     unsigned long long spans;
-    uint32_t queue2;    // queue of k_fused over the handed-on paths
     uint32_t queue3;    // queue of the large-grid dense kernel
     uint32_t dq2;       // paths handed on by the second dense instance
     uint32_t queue4;    // queue of the third dense instance
     uint32_t dq3;       // paths handed on by the third dense instance
-    uint32_t pad[51];
+    uint32_t pad[52];
 };
 
 __global__ void k_fused_reset(FusedCtl* c) {
@@ -100,7 +80,6 @@ __global__ void k_fused_reset(FusedCtl* c) {
         c->dq = 0;
         c->tiles = 0;
         c->spans = 0;
-        c->queue2 = 0;
         c->queue3 = 0;
         c->dq2 = 0;
         c->queue4 = 0;
@@ -148,20 +127,15 @@ __device__ inline uint32_t tile_rank(const S& s, int tx, int ty) {
 // instead of a dependent global load.
 struct LineWindow {
     float4 w0, w1;
-    uint32_t o0, o1;  // per-line increment offsets (emit walk)
     uint32_t base;
-    __device__ void load(const float4* lines, const uint32_t* off, uint32_t L, uint32_t b, int lane) {
+    __device__ void load(const float4* lines, uint32_t L, uint32_t b, int lane) {
         base = b;
         const uint32_t i0 = b + lane, i1 = b + 64 + lane;
         w0 = i0 < L ? lines[i0] : make_float4(0, 0, 0, 0);
         w1 = i1 < L ? lines[i1] : make_float4(0, 0, 0, 0);
-        if (off) {
-            o0 = i0 < L ? off[i0] : 0u;
-            o1 = i1 < L ? off[i1] : 0u;
-        }
     }
     // Fetches line `my` (must be in [base, base + 128)) for every lane.
-    __device__ float4 get(uint32_t my, uint32_t* o, bool with_off) const {
+    __device__ float4 get(uint32_t my) const {
         const uint32_t src = my - base;
         const int sl = (int)(src & 63u);
         float4 a, b;
@@ -173,21 +147,15 @@ struct LineWindow {
         b.y = __shfl(w1.y, sl, WAVE);
         b.z = __shfl(w1.z, sl, WAVE);
         b.w = __shfl(w1.w, sl, WAVE);
-        if (with_off) {
-            uint32_t x0 = __shfl(o0, sl, WAVE), x1 = __shfl(o1, sl, WAVE);
-            *o = src < 64 ? x0 : x1;
-        }
         return src < 64 ? a : b;
     }
     // Slides by 64 once `next` has passed the first window.
-    __device__ void advance(const float4* lines, const uint32_t* off, uint32_t L, uint32_t next, int lane) {
+    __device__ void advance(const float4* lines, uint32_t L, uint32_t next, int lane) {
         if (next >= base + 64) {
             w0 = w1;
-            o0 = o1;
             base += 64;
             const uint32_t i1 = base + 64 + lane;
             w1 = i1 < L ? lines[i1] : make_float4(0, 0, 0, 0);
-            if (off) o1 = i1 < L ? off[i1] : 0u;
         }
     }
 };
@@ -251,24 +219,23 @@ __device__ inline Xform adjoint_local_xform(const FusedIn& in, int64_t p, int32_
     return X;
 }
 
-template <int TC, bool ADJ>
-__device__ void fused_path(const FusedIn& in, const FusedOut& out, FusedCtl* ctl, uint32_t* deferred,
-                           uint8_t* sc, LdsState<TC>& s, int64_t p, const AdjArgs& adj, uint8_t* asc) {
+// One path of the adjoint, on one wave: its lines (to the wave's scratch), its
+// occupied tiles and spans as the f32 forward has them, then adjoint_backward.
+template <int TC>
+__device__ void adjoint_path(const FusedIn& in, FusedCtl* ctl, uint32_t* deferred, uint8_t* sc, LdsState<TC>& s,
+                             int64_t p, const AdjArgs& adj, uint8_t* asc) {
     const int lane = threadIdx.x;
-    const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
     float4* lines = reinterpret_cast<float4*>(sc);
-    uint32_t* incoff = reinterpret_cast<uint32_t*>(sc + (size_t)F_LCAP * 16);
-    float4* incs = reinterpret_cast<float4*>(sc + (size_t)F_LCAP * 16 + (size_t)(F_LCAP + 1) * 4 + 12);
 
     const int64_t vb = in.verb_off[p], ve = in.verb_off[p + 1];
     const int64_t pb = in.point_off[p], pe = in.point_off[p + 1];
     const int64_t wb = in.weight_off[p], we = in.weight_off[p + 1];
-    if (ADJ && (ve - vb > A_VCAP || pe - pb > A_PCAP)) {  // over one wave's limits whatever its lines are
+    if (ve - vb > A_VCAP || pe - pb > A_PCAP) {  // over one wave's limits whatever its lines are
         if (lane == 0) deferred[atomicAdd(&ctl->deferred, 1u)] = (uint32_t)p;  // (the adjoint's large path)
         return;
     }
     int32_t aox = 0, aoy = 0;
-    const Xform X = ADJ ? adjoint_local_xform(in, p, &aox, &aoy) : in.xf[p];
+    const Xform X = adjoint_local_xform(in, p, &aox, &aoy);
 
     // ---------------------------------------------------------- flatten
     uint32_t L = 0;
@@ -347,7 +314,7 @@ __device__ void fused_path(const FusedIn& in, const FusedOut& out, FusedCtl* ctl
             uint32_t o = L + n_incl - n;
             command_lines(c, [&](V2 a, V2 b) { lines[o++] = make_float4(a.x, a.y, b.x, b.y); });
         }
-        if (ADJ && valid && i - vb < A_VCAP) {
+        if (valid && i - vb < A_VCAP) {
             reinterpret_cast<uint32_t*>(asc + A_OFF_CMDOFF)[i - vb] = L + n_incl - n;
             if (i == ve - 1) reinterpret_cast<uint32_t*>(asc + A_OFF_CMDOFF)[i - vb + 1] = L + n_incl;
             for (int k = 0; k < np; k++)
@@ -409,21 +376,13 @@ __device__ void fused_path(const FusedIn& in, const FusedOut& out, FusedCtl* ctl
         for (uint32_t line = (uint32_t)lane; line < L; line += WAVE) {
             const float4 ln = lines[line];
             const V2 a = mk(ln.x, ln.y), point = mk(ln.z, ln.w);
-            uint32_t cnt = 0;
-            if (line_tiles(a, point, cnt, mark, cross)) {
-                incoff[line] = cnt;
-                continue;
-            }
-            if (veq(point, a)) {  // rasterizer.rs:73
-                incoff[line] = 0;
-                continue;
-            }
+            if (line_tiles(a, point, mark, cross)) continue;
+            if (veq(point, a)) continue;  // rasterizer.rs:73
             Dda d;
             dda_init(d, a, point);
             int16_t ty_prev = div8(d.y), cur_tx = div8(d.x), cur_ty = ty_prev;
             mark(cur_tx, cur_ty);
             for (uint32_t steps = 0;;) {
-                cnt++;
                 bool term = dda_step(d);
                 if (term) {  // rasterizer.rs:118-121
                     d.x = f2i16(floorf(point.x));
@@ -446,7 +405,6 @@ __device__ void fused_path(const FusedIn& in, const FusedOut& out, FusedCtl* ctl
                     mark(tx, ty);
                 }
             }
-            incoff[line] = cnt;
         }
     }
     __syncthreads();
@@ -483,58 +441,21 @@ __device__ void fused_path(const FusedIn& in, const FusedOut& out, FusedCtl* ctl
     }
     const uint32_t rsp_incl = wave_incl_scan(row_spans, OpAdd());
     const uint32_t NS = __shfl(rsp_incl, WAVE - 1, WAVE);
-    if (ADJ) {
-        if (NT > (uint32_t)A_TCAP || NS > (uint32_t)A_SCAP) {
-            if (lane == 0) deferred[atomicAdd(&ctl->deferred, 1u)] = (uint32_t)p;  // the large path
-            return;
-        }
-        if (row_lane && row_spans) {
-            uint32_t si = rsp_incl - row_spans;
-            int32_t wnd = w_before, w_prev = 0, prev = -1;
-            const uint32_t o = s.occ[lane];
-            uint32_t* sp = reinterpret_cast<uint32_t*>(asc + A_OFF_SPANS);
-            for (int x = 0; x < GW; x++) {
-                wnd += s.u.tsign[lane * F_GRID + x];
-                if ((o >> x) & 1u) {
-                    if (prev >= 0 && x > prev + 1 && w_prev != 0) {
-                        sp[2 * si] = (uint32_t)lane;                                  // grid row
-                        sp[2 * si + 1] = (uint32_t)(prev + 1) | ((uint32_t)x << 16);  // tile columns [a, b)
-                        si++;
-                    }
-                    prev = x;
-                    w_prev = wnd;
-                }
-            }
-        }
-    }
-    const uint32_t NT_out = NT ? NT : 1u;
-    unsigned long long tb = 0, sb = 0;
-    if (!ADJ && lane == 0) {
-        tb = atomicAdd(&ctl->tiles, (unsigned long long)NT_out);
-        sb = atomicAdd(&ctl->spans, (unsigned long long)NS);
-        out.pts[p] = (int64_t)tb;
-        out.ptc[p] = (int32_t)NT_out;
-        out.pss[p] = (int64_t)sb;
-        out.psc[p] = (int32_t)NS;
-    }
-    tb = __shfl(tb, 0, WAVE);
-    sb = __shfl(sb, 0, WAVE);
-    if (!ADJ && (tb + NT_out > (unsigned long long)out.tile_cap || sb + NS > (unsigned long long)out.span_cap)) {
-        if (lane == 0) atomicOr(&ctl->error, (uint32_t)ERR_CAPACITY);
+    if (NT > (uint32_t)A_TCAP || NS > (uint32_t)A_SCAP) {
+        if (lane == 0) deferred[atomicAdd(&ctl->deferred, 1u)] = (uint32_t)p;  // the large path
         return;
     }
-    if (!ADJ && row_lane && row_spans) {
-        uint64_t si = sb + (rsp_incl - row_spans);
+    if (row_lane && row_spans) {
+        uint32_t si = rsp_incl - row_spans;
         int32_t wnd = w_before, w_prev = 0, prev = -1;
         const uint32_t o = s.occ[lane];
-        const int32_t ty = ty0 + lane;
+        uint32_t* sp = reinterpret_cast<uint32_t*>(asc + A_OFF_SPANS);
         for (int x = 0; x < GW; x++) {
             wnd += s.u.tsign[lane * F_GRID + x];
             if ((o >> x) & 1u) {
                 if (prev >= 0 && x > prev + 1 && w_prev != 0) {
-                    out.span_xy[2 * si] = (int16_t)((tx0 + prev + 1) * TILE);
-                    out.span_xy[2 * si + 1] = (int16_t)(ty * TILE);
-                    out.span_w[si] = (uint16_t)((uint16_t)(x - prev - 1) * (uint16_t)TILE);
+                    sp[2 * si] = (uint32_t)lane;                                  // grid row
+                    sp[2 * si + 1] = (uint32_t)(prev + 1) | ((uint32_t)x << 16);  // tile columns [a, b)
                     si++;
                 }
                 prev = x;
@@ -542,222 +463,10 @@ __device__ void fused_path(const FusedIn& in, const FusedOut& out, FusedCtl* ctl
             }
         }
     }
-    if (ADJ) {
-        // (the adjoint takes its coverage from the f64 geometry: emitting and
-        // committing the f32 increments in front of it was half of its walks,
-        // 1,447 -> 1,137 us on 4,096 paths of 16 cubics)
-        adjoint_backward<TC>(in, adj, ctl, sc, asc, s, p, L, NT, NS, tx0, ty0, GW, GH);
-        return;
-    }
-    if (NT == 0) {  // no increments: one all-zero tile at (0, 0) (rasterizer.rs:193-198)
-        if (lane < 4) reinterpret_cast<uint4*>(out.tile_alpha + tb * 64)[lane] = make_uint4(0, 0, 0, 0);
-        if (out.tile_cov)
-            for (int k = lane; k < 64; k += WAVE) out.tile_cov[tb * 64 + k] = 0.0f;
-        if (lane == 0) {
-            out.tile_xy[2 * tb] = 0;
-            out.tile_xy[2 * tb + 1] = 0;
-        }
-        return;
-    }
-
-    // ------------------------------------------- increment offsets
-    {
-        uint32_t run = 0;
-        for (uint32_t b = 0; b < L; b += WAVE) {
-            uint32_t j = b + lane;
-            uint32_t c = j < L ? incoff[j] : 0u;
-            uint32_t ci = wave_incl_scan(c, OpAdd());
-            if (j < L) incoff[j] = run + ci - c;
-            run += __shfl(ci, WAVE - 1, WAVE);
-        }
-        if (lane == 0) incoff[L] = run;
-    }
-    __syncthreads();
-
-    // ------------------------------------- chunks of tiles: emit, commit
-    float carry = 0.0f;
-    int carry_row = -1;
-    for (uint32_t r0 = 0; r0 < NT; r0 += TC) {
-        const uint32_t nt = NT - r0 < (uint32_t)TC ? NT - r0 : (uint32_t)TC;
-        if ((uint32_t)lane < nt) {
-            uint32_t rank = r0 + lane;
-            int ty = 0;
-            while (ty + 1 < GH && s.row_rank[ty + 1] <= rank) ty++;
-            uint32_t k = rank - s.row_rank[ty];
-            uint32_t o = s.occ[ty];
-            for (uint32_t q = 0; q < k; q++) o &= o - 1;
-            int tx = __ffs(o) - 1;
-            s.chunk_tile[lane] = ((uint32_t)ty << 8) | (uint32_t)tx;
-        }
-        for (int k = lane; k < TC * F_TSTRIDE; k += WAVE) {
-            s.u.a.acc_a[k] = 0.0f;
-            s.u.a.acc_h[k] = 0.0f;
-        }
-        __syncthreads();
-        uint32_t l0 = 0;
-        while (l0 < L) {
-            // lines [l0, l1) whose increments fit the batch buffer
-            const uint32_t base = incoff[l0];
-            uint32_t lo = l0 + 1, hi = L;
-            while (lo < hi) {
-                uint32_t mid = (lo + hi + 1) >> 1;
-                if (incoff[mid] - base <= (uint32_t)F_ICAP) lo = mid;
-                else hi = mid - 1;
-            }
-            const uint32_t l1 = lo;
-            const uint32_t n_inc = incoff[l1] - base;
-            if (n_inc > (uint32_t)F_ICAP) {  // one line longer than the buffer: the grid cap rules it out
-                if (lane == 0) atomicOr(&ctl->error, (uint32_t)ERR_BBOX);
-                return;
-            }
-            // emit: lane per line, refilled as lines finish
-            {
-                uint32_t next = l0;
-                bool active = false;
-                Dda d;
-                uint32_t pos = 0;
-                int16_t cur_tx = 0, cur_ty = 0;
-                uint32_t slot_base = F_INVALID;
-                LineWindow win;
-                win.load(lines, incoff, l1, l0, lane);
-                while (next < l1 || __ballot(active)) {
-                    const uint64_t need = __ballot(!active);
-                    const uint32_t my = next + (uint32_t)__popcll(need & lt);
-                    float4 ln = make_float4(0, 0, 0, 0);
-                    uint32_t lo_off = 0;
-                    if (need && next < l1) ln = win.get(my, &lo_off, true);
-                    if (!active && my < l1) {
-                        V2 a = mk(ln.x, ln.y), b = mk(ln.z, ln.w);
-                        if (!veq(a, b)) {
-                            dda_init(d, a, b);
-                            pos = lo_off - base;
-                            cur_tx = (int16_t)0x7fff;
-                            cur_ty = (int16_t)0x7fff;
-                            active = true;
-                        }
-                    }
-                    next += (uint32_t)__popcll(need);
-                    win.advance(lines, incoff, l1, next, lane);
-                    if (active) {
-                        int16_t tx = div8(d.x), ty = div8(d.y);
-                        if (tx != cur_tx || ty != cur_ty) {
-                            cur_tx = tx;
-                            cur_ty = ty;
-                            uint32_t rank = tile_rank(s, tx - tx0, ty - ty0);
-                            slot_base = (rank - r0 < nt) ? (rank - r0) * F_TSTRIDE : F_INVALID;
-                        }
-                        float area, height;
-                        dda_increment(d, area, height);
-                        uint32_t key = slot_base == F_INVALID ? F_INVALID
-                                                              : slot_base + (uint32_t)(((d.y & 7) << 3) | (d.x & 7));
-                        incs[pos++] = make_float4(__uint_as_float(key), area, height, 0.0f);
-                        if (dda_step(d)) active = false;
-                    }
-                }
-            }
-            __syncthreads();
-            // commit in emission order
-            const float4 inv = make_float4(__uint_as_float(F_INVALID), 0.0f, 0.0f, 0.0f);
-            float4 pf0 = (uint32_t)lane < n_inc ? incs[lane] : inv;
-            float4 pf1 = (uint32_t)(lane + WAVE) < n_inc ? incs[lane + WAVE] : inv;
-            for (uint32_t cb = 0; cb < n_inc; cb += WAVE) {
-                const float4 v = pf0;
-                pf0 = pf1;
-                const uint32_t jn = cb + 2 * WAVE + lane;
-                pf1 = jn < n_inc ? incs[jn] : inv;
-                const uint32_t key = __float_as_uint(v.x);
-                const bool valid = key != F_INVALID;
-                uint64_t match = __ballot(valid);
-#pragma unroll
-                for (int b = 0; b < 12; b++) {
-                    const bool bit = (key >> b) & 1u;
-                    const uint64_t m = __ballot(bit);
-                    match &= bit ? m : ~m;
-                }
-                const int rank = __popcll(match & lt);
-                for (int r = 0;; r++) {
-                    if (valid && rank == r) {
-                        s.u.a.acc_a[key] += v.y;
-                        s.u.a.acc_h[key] += v.z;
-                    }
-                    if (!__ballot(valid && rank > r)) break;
-                }
-            }
-            __syncthreads();
-            l0 = l1;
-        }
-        // row carry, one lane per pixel row, sequential over the chunk's tiles
-        if (lane < 8) {
-            for (uint32_t t = 0; t < nt; t++) {
-                int ty = (int)(s.chunk_tile[t] >> 8);
-                if (ty != carry_row) {
-                    carry = 0.0f;
-                    carry_row = ty;
-                }
-                s.u.a.cin[t * 8 + lane] = carry;
-#pragma unroll
-                for (int x = 0; x < 8; x++) carry += s.u.a.acc_h[t * F_TSTRIDE + lane * 8 + x];
-            }
-        }
-        __syncthreads();
-        // quantise and store (rasterizer.rs:231-241)
-        if ((uint32_t)lane < nt) {
-            const int t = lane;
-            const int ty = (int)(s.chunk_tile[t] >> 8), tx = (int)(s.chunk_tile[t] & 0xffu);
-            uint32_t words[16];
-#pragma unroll
-            for (int y = 0; y < 8; y++) {
-                float accum = s.u.a.cin[t * 8 + y];
-                uint32_t w0 = 0, w1 = 0;
-#pragma unroll
-                for (int x = 0; x < 8; x++) {
-                    const int k = t * F_TSTRIDE + y * 8 + x;
-                    if (out.tile_cov)
-                        out.tile_cov[(tb + r0 + (uint32_t)t) * 64 + y * 8 + x] = fminf(fabsf(accum + s.u.a.acc_a[k]), 1.0f);
-                    float v = fminf(fabsf(accum + s.u.a.acc_a[k]) * 256.0f, 255.0f);
-                    uint32_t b = (uint32_t)v;
-                    if (x < 4) w0 |= b << (8 * x);
-                    else w1 |= b << (8 * (x - 4));
-                    accum += s.u.a.acc_h[k];
-                }
-                words[2 * y] = w0;
-                words[2 * y + 1] = w1;
-            }
-            const uint64_t ti = tb + r0 + (uint32_t)t;
-            uint4* dst = reinterpret_cast<uint4*>(out.tile_alpha + ti * 64);
-            dst[0] = make_uint4(words[0], words[1], words[2], words[3]);
-            dst[1] = make_uint4(words[4], words[5], words[6], words[7]);
-            dst[2] = make_uint4(words[8], words[9], words[10], words[11]);
-            dst[3] = make_uint4(words[12], words[13], words[14], words[15]);
-            out.tile_xy[2 * ti] = (int16_t)((tx0 + tx) * TILE);
-            out.tile_xy[2 * ti + 1] = (int16_t)((ty0 + ty) * TILE);
-        }
-        __syncthreads();
-    }
-}
-
-template <int TC>
-__global__ __launch_bounds__(WAVE) void k_fused(FusedIn in, FusedOut out, FusedCtl* ctl, uint32_t* deferred,
-                                                uint8_t* scratch, uint32_t gran) {
-    __shared__ LdsState<TC> s;
-    uint8_t* sc = scratch + (size_t)blockIdx.x * F_SCRATCH;
-    const int64_t n = in.ids ? (int64_t)*in.n_ids : in.n_paths;
-    if (n == 0) return;  // nothing handed on (the common case behind the dense kernels)
-    if (in.ids && n > (int64_t)in.defer_above) {
-        for (int64_t q = (int64_t)blockIdx.x * WAVE + threadIdx.x; q < n; q += (int64_t)gridDim.x * WAVE)
-            deferred[atomicAdd(&ctl->deferred, 1u)] = in.ids[q];
-        return;
-    }
-    for (;;) {
-        uint32_t base = 0;
-        if (threadIdx.x == 0) base = atomicAdd(in.ids ? &ctl->queue2 : &ctl->queue, gran);
-        base = __shfl(base, 0, WAVE);
-        if ((int64_t)base >= n) break;
-        const int64_t end = std::min<int64_t>((int64_t)base + gran, n);
-        for (int64_t q = base; q < end; q++)
-            fused_path<TC, false>(in, out, ctl, deferred, sc, s, in.ids ? (int64_t)in.ids[q] : q, AdjArgs{},
-                                  nullptr);
-    }
+    // (the adjoint takes its coverage from the f64 geometry: emitting and
+    // committing the f32 increments in front of it was half of its walks,
+    // 1,447 -> 1,137 us on 4,096 paths of 16 cubics)
+    adjoint_backward<TC>(in, adj, ctl, sc, asc, s, p, L, NT, NS, tx0, ty0, GW, GH);
 }
 
 #include "adjoint.inc"
@@ -799,12 +508,10 @@ __global__ void k_scatter_ranges(const uint32_t* ids, uint32_t n, const int64_t*
 }
 
 struct BatchedState {
-    DBuf scratch, ascratch, ctl, deferred, dense_ids, dense_ids2, dense_ids3;
+    DBuf scratch, ascratch, ctl, deferred, dense_ids, dense_ids2, dense_ids3, d_sizes, d_pack;
     DBuf large_cmd, large_grid;  // the large-path adjoint's scratch
-    DBuf g_verbs, g_points, g_weights, g_voff, g_poff, g_woff, g_xf, g_ts, g_tc, g_ss, g_sc;
-    int n_waves = 0;
-    uint32_t gran = 1;
-    // graph of (reset, fused) for the last argument set
+    DBuf g_verbs, g_points, g_weights, g_xf, g_ts, g_tc, g_ss, g_sc;
+    // graph of (reset, dense kernels) for the last argument set
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     std::vector<uint8_t> graph_key;
@@ -814,21 +521,46 @@ struct BatchedState {
     }
 };
 
-int run_batched(Context* ctx, const SegInput& in, OutputDesc& out, hipStream_t s, int waves_per_cu, int gran,
-                int tiles_per_chunk, bool use_graph) {
+// The plain pipeline in passes of bounded scratch: a call that took the batched
+// pipeline's fixed scratch before must not need the plain one's tens of gigabytes
+// for a large batch.  About 0.8 GB at the first limits, 0.1 GB at the second,
+// which a pass falls back to when memory is short; a single path over them still
+// gets the context's own limits.
+static int run_plain_bounded(Context* ctx, const SegInput& in, OutputDesc& out, hipStream_t s) {
+    const OutputDesc asked = out;
+    int st = run_plain(ctx, in, out, s, false, (int64_t)1 << 23, (int64_t)1 << 24);
+    if (st == -2) {
+        (void)hipGetLastError();
+        out = asked;
+        st = run_plain(ctx, in, out, s, false, (int64_t)1 << 20, (int64_t)1 << 21);
+    }
+    return st;
+}
+
+// The handed-on paths' command, point and weight counts.
+struct DeferSize {
+    int64_t path, nv, np, nw;
+};
+__global__ void k_defer_sizes(FusedIn in, const uint32_t* ids, uint32_t n, DeferSize* out) {
+    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= n) return;
+    const int64_t p = ids[k];
+    out[k] = DeferSize{p, in.verb_off[p + 1] - in.verb_off[p], in.point_off[p + 1] - in.point_off[p],
+                       in.weight_off[p + 1] - in.weight_off[p]};
+}
+
+int run_batched(Context* ctx, const SegInput& in, OutputDesc& out, hipStream_t s, bool use_graph) {
     if (!ctx->batched) ctx->batched = new BatchedState();
     BatchedState* B = reinterpret_cast<BatchedState*>(ctx->batched);
     const int64_t NP = in.n_paths;
     out.n_tiles = out.n_spans = 0;
     if (NP <= 0) return 0;
+    if (!ctx->dense) return run_plain_bounded(ctx, in, out, s);
     int dev = 0;
     HIPCHK_RET(hipGetDevice(&dev));
     int cus = 0;
     HIPCHK_RET(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    const int n_waves = std::max(1, cus * std::max(1, waves_per_cu));
-    HIPCHK_RET(B->scratch.ensure((size_t)n_waves * F_SCRATCH));
     HIPCHK_RET(B->ctl.ensure(sizeof(FusedCtl)));
-    HIPCHK_RET(B->deferred.ensure((size_t)NP * 4));
     if (!ctx->host_pinned) HIPCHK_RET(hipHostMalloc(&ctx->host_pinned, 4096));
     FusedIn fi;
     fi.n_paths = NP;
@@ -854,48 +586,36 @@ int run_batched(Context* ctx, const SegInput& in, OutputDesc& out, hipStream_t s
     fo.pss = out.path_span_start;
     fo.psc = out.path_span_count;
     FusedCtl* ctl = B->ctl.as<FusedCtl>();
-    uint32_t* deferred = B->deferred.as<uint32_t>();
-    uint8_t* scratch = B->scratch.as<uint8_t>();
-    const uint32_t g = (uint32_t)std::max(1, gran);
-    const bool tc16 = tiles_per_chunk <= 16;
-    const bool dense = ctx->dense;
     const int dnw = ctx->dense_waves == 2 ? 2 : (ctx->dense_waves == 8 ? 8 : 4);
     const int n_groups = std::max(1, cus * std::max(1, ctx->dense_groups_per_cu));
-    const int n_small = dense ? cus * std::max(0, ctx->dense_small_groups) : 0;
-    const int n_large = (dense && ctx->dense_large) ? cus : 0;
+    const int n_small = cus * std::max(0, ctx->dense_small_groups);
+    const int n_large = ctx->dense_large ? cus : 0;
     // The dense instances run one after another, each over the paths the one
-    // before handed on: [small grids, 32 tiles] -> 64 tiles -> [256 tiles], then
-    // the ordered kernel over what is left.
+    // before handed on: [small grids, 32 tiles] -> 64 tiles -> [256 tiles]; what is
+    // left goes to the plain pipeline.
     enum { D_SMALL, D_MAIN, D_LARGE };
     int stages[3], n_stages = 0;
-    if (dense) {
-        if (n_small) stages[n_stages++] = D_SMALL;
-        stages[n_stages++] = D_MAIN;
-        if (n_large) stages[n_stages++] = D_LARGE;
-    }
-    uint32_t* lists[3] = {nullptr, nullptr, nullptr};
+    if (n_small) stages[n_stages++] = D_SMALL;
+    stages[n_stages++] = D_MAIN;
+    if (n_large) stages[n_stages++] = D_LARGE;
+    HIPCHK_RET(B->dense_ids.ensure((size_t)NP * 4));
+    if (n_stages > 1) HIPCHK_RET(B->dense_ids2.ensure((size_t)NP * 4));
+    if (n_stages > 2) HIPCHK_RET(B->dense_ids3.ensure((size_t)NP * 4));
+    uint32_t* lists[3] = {B->dense_ids.as<uint32_t>(), B->dense_ids2.as<uint32_t>(), B->dense_ids3.as<uint32_t>()};
     uint32_t* counts[3] = {&ctl->dq, &ctl->dq2, &ctl->dq3};
     uint32_t* queues[3] = {&ctl->queue, &ctl->queue3, &ctl->queue4};
-    FusedIn fin[4] = {fi, fi, fi, fi};  // stage i reads fin[i]; k_fused reads fin[n_stages]
-    if (dense) {
-        HIPCHK_RET(B->dense_ids.ensure((size_t)NP * 4));
-        HIPCHK_RET(B->dense_ids2.ensure((size_t)NP * 4));
-        if (n_stages > 2) HIPCHK_RET(B->dense_ids3.ensure((size_t)NP * 4));
-        lists[0] = B->dense_ids.as<uint32_t>();
-        lists[1] = B->dense_ids2.as<uint32_t>();
-        lists[2] = B->dense_ids3.as<uint32_t>();
-        for (int i = 1; i <= n_stages; i++) {
-            fin[i].ids = lists[i - 1];
-            fin[i].n_ids = counts[i - 1];
-        }
-        fin[n_stages].defer_above = F_DEFER_ABOVE;
+    FusedIn fin[3] = {fi, fi, fi};  // stage i reads fin[i]
+    for (int i = 1; i < n_stages; i++) {
+        fin[i].ids = lists[i - 1];
+        fin[i].n_ids = counts[i - 1];
     }
+    uint32_t* deferred = lists[n_stages - 1];
     const bool timing = ctx->timing;
     if (timing) {
         for (auto& e : ctx->ev)
             if (!e) HIPCHK_RET(hipEventCreate(&e));
     }
-    // timing without a graph brackets the dense kernels and k_fused with events
+    // timing without a graph brackets the dense kernels with events
     auto enqueue = [&](hipStream_t st, bool ev) {
         hipLaunchKernelGGL(k_fused_reset, dim3(1), dim3(64), 0, st, ctl);
         if (ev) (void)hipEventRecord(ctx->ev[0], st);
@@ -917,25 +637,25 @@ int run_batched(Context* ctx, const SegInput& in, OutputDesc& out, hipStream_t s
                 hipLaunchKernelGGL((k_dense<4, 64>), dim3(n_groups), dim3(4 * WAVE), 0, st, f, fo, ctl, queues[i],
                                    lists[i], counts[i]);
         }
-        if (dense && ev) (void)hipEventRecord(ctx->ev[2], st);
-        const FusedIn& f = fin[n_stages];
-        if (tc16) hipLaunchKernelGGL(k_fused<16>, dim3(n_waves), dim3(WAVE), 0, st, f, fo, ctl, deferred, scratch, g);
-        else hipLaunchKernelGGL(k_fused<32>, dim3(n_waves), dim3(WAVE), 0, st, f, fo, ctl, deferred, scratch, g);
         if (ev) (void)hipEventRecord(ctx->ev[1], st);
     };
+    bool replay = false;
     if (use_graph) {
-        std::vector<uint8_t> key(sizeof(fi) + sizeof(fo) + 41);
-        key.back() = tc16 ? 1 : 0;
-        memcpy(key.data(), &fi, sizeof(fi));
-        memcpy(key.data() + sizeof(fi), &fo, sizeof(fo));
-        memcpy(key.data() + sizeof(fi) + sizeof(fo), &n_waves, 4);
-        memcpy(key.data() + sizeof(fi) + sizeof(fo) + 4, &g, 4);
-        memcpy(key.data() + sizeof(fi) + sizeof(fo) + 8, &scratch, 8);
-        const int dkey = dense ? (dnw << 16) | n_groups : 0;
-        memcpy(key.data() + sizeof(fi) + sizeof(fo) + 24, &dkey, 4);
-        memcpy(key.data() + sizeof(fi) + sizeof(fo) + 28, &n_small, 4);
-        memcpy(key.data() + sizeof(fi) + sizeof(fo) + 32, &n_large, 4);
-        if (!B->exec || key != B->graph_key) {
+        std::vector<uint8_t> key(sizeof(fi) + sizeof(fo) + 40, 0);
+        uint8_t* at = key.data();
+        auto put = [&](const void* p, size_t n) {
+            memcpy(at, p, n);
+            at += n;
+        };
+        put(&fi, sizeof(fi));
+        put(&fo, sizeof(fo));
+        put(lists, sizeof(lists));
+        put(&dnw, 4);
+        put(&n_groups, 4);
+        put(&n_small, 4);
+        put(&n_large, 4);
+        replay = B->exec && key == B->graph_key;
+        if (!replay) {
             if (B->exec) (void)hipGraphExecDestroy(B->exec);
             if (B->graph) (void)hipGraphDestroy(B->graph);
             B->exec = nullptr;
@@ -949,7 +669,10 @@ int run_batched(Context* ctx, const SegInput& in, OutputDesc& out, hipStream_t s
             HIPCHK_RET(e);
             HIPCHK_RET(hipGraphInstantiate(&B->exec, B->graph, nullptr, nullptr, 0));
             B->graph_key = key;
+            replay = true;
         }
+    }
+    if (replay) {
         if (timing) HIPCHK_RET(hipEventRecord(ctx->ev[0], s));
         HIPCHK_RET(hipGraphLaunch(B->exec, s));
         if (timing) HIPCHK_RET(hipEventRecord(ctx->ev[1], s));
@@ -961,25 +684,16 @@ int run_batched(Context* ctx, const SegInput& in, OutputDesc& out, hipStream_t s
     HIPCHK_RET(hipMemcpyAsync(hc, ctl, sizeof(FusedCtl), hipMemcpyDeviceToHost, s));
     HIPCHK_RET(hipStreamSynchronize(s));
     if (timing) {
-        // graph: the whole launch; direct: k_dense and k_fused separately
+        // graph: the whole launch; direct: the dense kernels
         float ms = 0;
-        if (use_graph) {
+        if (replay) {
             HIPCHK_RET(hipEventElapsedTime(&ms, ctx->ev[0], ctx->ev[1]));
             auto& t = ctx->timings["batched_graph"];
             t.first += ms;
             t.second += 1;
-        } else if (dense) {
-            HIPCHK_RET(hipEventElapsedTime(&ms, ctx->ev[0], ctx->ev[2]));
-            auto& t = ctx->timings["k_dense"];
-            t.first += ms;
-            t.second += 1;
-            HIPCHK_RET(hipEventElapsedTime(&ms, ctx->ev[2], ctx->ev[1]));
-            auto& t2 = ctx->timings["k_fused"];
-            t2.first += ms;
-            t2.second += 1;
         } else {
             HIPCHK_RET(hipEventElapsedTime(&ms, ctx->ev[0], ctx->ev[1]));
-            auto& t = ctx->timings["k_fused"];
+            auto& t = ctx->timings["k_dense"];
             t.first += ms;
             t.second += 1;
         }
@@ -988,45 +702,47 @@ int run_batched(Context* ctx, const SegInput& in, OutputDesc& out, hipStream_t s
     if (hc->error & ERR_FLATTEN) return -5;
     if (hc->error & ERR_BBOX) return -3;
     const int64_t Tf = (int64_t)hc->tiles, Sf = (int64_t)hc->spans;
-    const uint32_t nd = hc->deferred;
+    const uint32_t nd = n_stages == 1 ? hc->dq : (n_stages == 2 ? hc->dq2 : hc->dq3);
     int64_t Tp = 0, Sp = 0;
     int st = 0;
     if (nd > 0) {
         // compact the deferred paths and run the plain pipeline on them
-        std::vector<uint32_t> ids(nd);
-        HIPCHK_RET(hipMemcpy(ids.data(), deferred, nd * 4, hipMemcpyDeviceToHost));
-        std::sort(ids.begin(), ids.end());
-        std::vector<int64_t> voff(NP + 1), poff(NP + 1), woff(NP + 1);
-        HIPCHK_RET(hipMemcpy(voff.data(), in.seg_verb_off, (NP + 1) * 8, hipMemcpyDeviceToHost));
-        HIPCHK_RET(hipMemcpy(poff.data(), in.seg_point_off, (NP + 1) * 8, hipMemcpyDeviceToHost));
-        HIPCHK_RET(hipMemcpy(woff.data(), in.seg_weight_off, (NP + 1) * 8, hipMemcpyDeviceToHost));
-        std::vector<int64_t> dv(nd + 1, 0), dp(nd + 1, 0), dw(nd + 1, 0);
+        HIPCHK_RET(B->d_sizes.ensure((size_t)nd * sizeof(DeferSize)));
+        hipLaunchKernelGGL(k_defer_sizes, dim3((nd + 255) / 256), dim3(256), 0, s, fi, deferred, nd,
+                           B->d_sizes.as<DeferSize>());
+        HIPCHK_RET(hipGetLastError());
+        std::vector<DeferSize> sz(nd);
+        HIPCHK_RET(hipMemcpyAsync(sz.data(), B->d_sizes.p, (size_t)nd * sizeof(DeferSize), hipMemcpyDeviceToHost, s));
+        HIPCHK_RET(hipStreamSynchronize(s));
+        std::sort(sz.begin(), sz.end(), [](const DeferSize& x, const DeferSize& y) { return x.path < y.path; });
+        // offsets of the compact batch and the paths, in one upload: voff, poff, woff | ids
+        const size_t no = (size_t)nd + 1;
+        std::vector<int64_t> pack(3 * no + (nd + 1) / 2, 0);
+        int64_t *dv = pack.data(), *dp = dv + no, *dw = dp + no;
+        uint32_t* ids = reinterpret_cast<uint32_t*>(dw + no);
         for (uint32_t k = 0; k < nd; k++) {
-            uint32_t p = ids[k];
-            dv[k + 1] = dv[k] + voff[p + 1] - voff[p];
-            dp[k + 1] = dp[k] + poff[p + 1] - poff[p];
-            dw[k + 1] = dw[k] + woff[p + 1] - woff[p];
+            dv[k + 1] = dv[k] + sz[k].nv;
+            dp[k + 1] = dp[k] + sz[k].np;
+            dw[k + 1] = dw[k] + sz[k].nw;
+            ids[k] = (uint32_t)sz[k].path;
         }
         HIPCHK_RET(B->g_verbs.ensure(std::max<int64_t>(dv[nd], 1)));
         HIPCHK_RET(B->g_points.ensure(std::max<int64_t>(dp[nd], 1) * 8));
         HIPCHK_RET(B->g_weights.ensure(std::max<int64_t>(dw[nd], 1) * 4));
-        HIPCHK_RET(B->g_voff.ensure((nd + 1) * 8));
-        HIPCHK_RET(B->g_poff.ensure((nd + 1) * 8));
-        HIPCHK_RET(B->g_woff.ensure((nd + 1) * 8));
+        HIPCHK_RET(B->d_pack.ensure(pack.size() * 8));
         HIPCHK_RET(B->g_xf.ensure(nd * sizeof(Xform)));
         HIPCHK_RET(B->g_ts.ensure(nd * 8));
         HIPCHK_RET(B->g_tc.ensure(nd * 4));
         HIPCHK_RET(B->g_ss.ensure(nd * 8));
         HIPCHK_RET(B->g_sc.ensure(nd * 4));
-        HIPCHK_RET(hipMemcpyAsync(deferred, ids.data(), nd * 4, hipMemcpyHostToDevice, s));
-        HIPCHK_RET(hipMemcpyAsync(B->g_voff.p, dv.data(), (nd + 1) * 8, hipMemcpyHostToDevice, s));
-        HIPCHK_RET(hipMemcpyAsync(B->g_poff.p, dp.data(), (nd + 1) * 8, hipMemcpyHostToDevice, s));
-        HIPCHK_RET(hipMemcpyAsync(B->g_woff.p, dw.data(), (nd + 1) * 8, hipMemcpyHostToDevice, s));
+        HIPCHK_RET(hipMemcpyAsync(B->d_pack.p, pack.data(), pack.size() * 8, hipMemcpyHostToDevice, s));
+        const int64_t* g_voff = B->d_pack.as<int64_t>();
+        const int64_t *g_poff = g_voff + no, *g_woff = g_poff + no;
+        deferred = reinterpret_cast<uint32_t*>(B->d_pack.as<int64_t>() + 3 * no);
         const uint32_t slices = std::max<uint32_t>(1, std::min<uint32_t>(64, 4096 / nd));
         hipLaunchKernelGGL(k_gather_paths, dim3(std::min<uint32_t>(nd, 4096), slices), dim3(256), 0, s, fi, deferred, nd,
-                           B->g_voff.as<int64_t>(), B->g_poff.as<int64_t>(), B->g_woff.as<int64_t>(),
-                           B->g_verbs.as<uint8_t>(), B->g_points.as<float>(), B->g_weights.as<float>(),
-                           B->g_xf.as<Xform>());
+                           g_voff, g_poff, g_woff, B->g_verbs.as<uint8_t>(), B->g_points.as<float>(),
+                           B->g_weights.as<float>(), B->g_xf.as<Xform>());
         HIPCHK_RET(hipGetLastError());
         SegInput si;
         si.n_segs = nd;
@@ -1034,9 +750,9 @@ int run_batched(Context* ctx, const SegInput& in, OutputDesc& out, hipStream_t s
         si.verbs = B->g_verbs.as<uint8_t>();
         si.points = B->g_points.as<float>();
         si.weights = B->g_weights.as<float>();
-        si.seg_verb_off = B->g_voff.as<int64_t>();
-        si.seg_point_off = B->g_poff.as<int64_t>();
-        si.seg_weight_off = B->g_woff.as<int64_t>();
+        si.seg_verb_off = g_voff;
+        si.seg_point_off = g_poff;
+        si.seg_weight_off = g_woff;
         si.seg_xf = B->g_xf.as<Xform>();
         si.n_verbs = dv[nd];
         si.n_points = dp[nd];
@@ -1055,8 +771,8 @@ int run_batched(Context* ctx, const SegInput& in, OutputDesc& out, hipStream_t s
         od.path_span_start = B->g_ss.as<int64_t>();
         od.path_span_count = B->g_sc.as<int32_t>();
         // under the dense kernels' 1-LSB contract the handed-on paths take the
-        // unordered tile stage; with them off the plain pipeline stays exact
-        st = run_plain(ctx, si, od, s, dense);
+        // unordered tile stage
+        st = run_plain(ctx, si, od, s, true);
         Tp = od.n_tiles;
         Sp = od.n_spans;
         if (st == 0) {

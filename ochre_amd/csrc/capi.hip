@@ -187,8 +187,7 @@ int ochre_rasterize_batched(ochre_context* ctx, const ochre_path_batch* in, ochr
     std::lock_guard<std::mutex> lk(ctx->mu);
     if (hipSetDevice(ctx->c.device) != hipSuccess) return OCHRE_ERR_DEVICE;
     OutputDesc od = to_output(out);
-    st = run_batched(&ctx->c, si, od, reinterpret_cast<hipStream_t>(stream), ctx->c.batched_waves_per_cu,
-                     ctx->c.batched_gran, ctx->c.batched_tc, ctx->c.batched_graph);
+    st = run_batched(&ctx->c, si, od, reinterpret_cast<hipStream_t>(stream), ctx->c.batched_graph);
     out->n_tiles = od.n_tiles;
     out->n_spans = od.n_spans;
     return st;
@@ -357,9 +356,7 @@ int ochre_coverage_adjoint(ochre_context* ctx, const ochre_path_batch* in, const
     t.span_count = target->span_count;
     t.span_xy = target->span_xy;
     t.span_w = target->span_width;
-    // The adjoint's own launch shape, not the batched call's tuned one (which
-    // is tuned for the ordered kernel behind the dense ones and may leave it a
-    // wave per CU): on 4,096 16-cubic glyphs 32-tile chunks, a path per pop and
+    // The adjoint's own launch shape: on 4,096 16-cubic glyphs 32-tile chunks, a path per pop and
     // 8 or more waves per CU measured 1.58-1.61 ms, 16-tile chunks 2.37-2.42,
     // one wave per CU 6.6-9.8 ms.
     return run_adjoint(&ctx->c, si, t, loss, d_points, d_transforms, reinterpret_cast<hipStream_t>(stream), 8, 1,
@@ -375,23 +372,21 @@ int ochre_autotune_batched(ochre_context* ctx, const ochre_path_batch* in, ochre
     std::lock_guard<std::mutex> lk(ctx->mu);
     if (hipSetDevice(ctx->c.device) != hipSuccess) return OCHRE_ERR_DEVICE;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    static const int waves[] = {2, 3, 4, 6, 8, 12};
-    static const int grans[] = {1, 2, 4, 8};
-    static const int tcs[] = {16, 32};
     static const int dgroups[] = {1, 2, 3, 4};
     static const int dwaves[] = {2, 4, 8};
     ochre_batched_tuning best{ctx->c.batched_waves_per_cu, ctx->c.batched_gran, ctx->c.batched_tc, 1e30f, 0, 0, 0, 0};
     int best_dg = ctx->c.dense_groups_per_cu, best_dw = ctx->c.dense_waves;
     int k = 0;
-    auto measure = [&](int w, int g, int tc, float* ms_out) -> int {
+    auto measure = [&](float* ms_out) -> int {
         OutputDesc od = to_output(out);
-        // warm-up (also captures the graph for this configuration)
-        int rc = run_batched(&ctx->c, si, od, s, w, g, tc, true);
+        // warm-up (the second call captures the graph for this configuration)
+        int rc = run_batched(&ctx->c, si, od, s, true);
+        if (!rc) rc = run_batched(&ctx->c, si, od, s, true);
         if (rc) return rc;
         std::vector<double> t;
         for (int r = 0; r < reps; r++) {
             auto t0 = std::chrono::steady_clock::now();
-            rc = run_batched(&ctx->c, si, od, s, w, g, tc, true);
+            rc = run_batched(&ctx->c, si, od, s, true);
             if (rc) return rc;
             t.push_back(std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count());
         }
@@ -400,16 +395,13 @@ int ochre_autotune_batched(ochre_context* ctx, const ochre_path_batch* in, ochre
         return 0;
     };
     if (ctx->c.dense) {
-        // the ordered kernel only sees the paths the dense one hands on:
-        // tune the dense launch shape, with waves/CU and tiles per chunk
-        // encoded as (groups per CU, waves per group) in the results
         for (int dg : dgroups)
             for (int dw : dwaves) {
                 if (dw == 8 && dg > 2) continue;  // 16 waves of 128 registers fill a CU
                 ctx->c.dense_groups_per_cu = dg;
                 ctx->c.dense_waves = dw;
                 float ms = 0;
-                st = measure(best.waves_per_cu, best.paths_per_pop, best.tiles_per_chunk, &ms);
+                st = measure(&ms);
                 if (st) return st;
                 if (results && k < max_results)
                     results[k] = ochre_batched_tuning{best.waves_per_cu, best.paths_per_pop, best.tiles_per_chunk, ms,
@@ -428,7 +420,7 @@ int ochre_autotune_batched(ochre_context* ctx, const ochre_path_batch* in, ochre
         for (int sg : {0, 4, 6, 8}) {
             ctx->c.dense_small_groups = sg;
             float ms = 0;
-            st = measure(best.waves_per_cu, best.paths_per_pop, best.tiles_per_chunk, &ms);
+            st = measure(&ms);
             if (st) return st;
             if (results && k < max_results)
                 results[k] = ochre_batched_tuning{best.waves_per_cu, best.paths_per_pop, best.tiles_per_chunk, ms,
@@ -445,7 +437,7 @@ int ochre_autotune_batched(ochre_context* ctx, const ochre_path_batch* in, ochre
         for (int lg : {0, 1}) {
             ctx->c.dense_large = lg;
             float ms = 0;
-            st = measure(best.waves_per_cu, best.paths_per_pop, best.tiles_per_chunk, &ms);
+            st = measure(&ms);
             if (st) return st;
             if (results && k < max_results)
                 results[k] = ochre_batched_tuning{best.waves_per_cu, best.paths_per_pop, best.tiles_per_chunk, ms,
@@ -457,37 +449,15 @@ int ochre_autotune_batched(ochre_context* ctx, const ochre_path_batch* in, ochre
             }
         }
         ctx->c.dense_large = best_large;
-        // then the persistent grid of the ordered kernel behind them, which
-        // only works through the paths the dense kernel hands on
-        for (int w : {1, 2, 4, 8}) {
-            float ms = 0;
-            st = measure(w, best.paths_per_pop, best.tiles_per_chunk, &ms);
-            if (st) return st;
-            if (results && k < max_results)
-                results[k] = ochre_batched_tuning{w, best.paths_per_pop, best.tiles_per_chunk, ms, best_dg, best_dw,
-                                                  ctx->c.dense_small_groups, ctx->c.dense_large};
-            k++;
-            if (ms < best.ms) {
-                best.ms = ms;
-                best.waves_per_cu = w;
-            }
-        }
-    } else {
-        for (int w : waves)
-            for (int g : grans)
-                for (int tc : tcs) {
-                    float ms = 0;
-                    st = measure(w, g, tc, &ms);
-                    if (st) return st;
-                    if (results && k < max_results) results[k] = ochre_batched_tuning{w, g, tc, ms, 0, 0, 0, 0};
-                    k++;
-                    if (ms < best.ms) best = ochre_batched_tuning{w, g, tc, ms, 0, 0, 0, 0};
-                }
+    } else {  // the plain pipeline has no launch shape to choose
+        float ms = 0;
+        st = measure(&ms);
+        if (st) return st;
+        if (results && k < max_results)
+            results[k] = ochre_batched_tuning{best.waves_per_cu, best.paths_per_pop, best.tiles_per_chunk, ms, 0, 0, 0, 0};
+        k++;
     }
     if (n_results) *n_results = k;
-    ctx->c.batched_waves_per_cu = best.waves_per_cu;
-    ctx->c.batched_gran = best.paths_per_pop;
-    ctx->c.batched_tc = best.tiles_per_chunk;
     ctx->c.batched_graph = true;
     return OCHRE_OK;
 }
@@ -1053,8 +1023,7 @@ int ochre_rasterizer_finish(ochre_rasterizer* r, const ochre_tile_builder* build
                 s1.path_seg_off = nullptr;
                 const bool dense = ctx->c.dense;
                 ctx->c.dense = false;
-                st = run_batched(&ctx->c, s1, od, s, ctx->c.batched_waves_per_cu, ctx->c.batched_gran,
-                                 ctx->c.batched_tc, false);
+                st = run_batched(&ctx->c, s1, od, s, false);
                 ctx->c.dense = dense;
             } else {
                 st = run_plain(&ctx->c, si, od, s);
@@ -1186,8 +1155,7 @@ static int finish_draws(ochre_rasterizer* const* rs, size_t m, const ochre_tile_
         od.path_span_count = dp->psc.as<int32_t>();
         st = any_stroke ? run_stroke(&ctx->c, si, static_cast<const float*>(dv[8]),
                                      static_cast<const uint8_t*>(dv[7]), od, s, true)
-                        : run_batched(&ctx->c, si, od, s, ctx->c.batched_waves_per_cu, ctx->c.batched_gran,
-                                      ctx->c.batched_tc, false);
+                        : run_batched(&ctx->c, si, od, s, false);
         if (st != OCHRE_ERR_CAPACITY) break;
         tcap = od.n_tiles;
         scap = od.n_spans;

@@ -132,6 +132,7 @@ struct Context {
     DBuf u_pwbase, u_rwbase, u_bcnt, u_bbeg, u_bcur;  // unordered tile stage: window buckets
     double split_ratio = 2.0;  // how far the last pass that had to split was over its limits
     int64_t max_lines = PLAIN_MAX_LINES, max_entries = PLAIN_MAX_ENTRIES;  // per-pass limits (lowered by tests)
+    int64_t pass_lines = PLAIN_MAX_LINES, pass_entries = PLAIN_MAX_ENTRIES;  // of the current pass
     // host staging
     void* host_pinned = nullptr;
     // timing
@@ -144,13 +145,13 @@ struct Context {
     int batched_gran = 2;
     int batched_tc = 32;
     bool batched_graph = true;
-    // dense single-walk kernel in front of the ordered one: on/off, resident
-    // workgroups per CU, waves per workgroup (2 or 4)
+    // dense single-walk kernel: on/off, resident workgroups per CU, waves per
+    // workgroup (2, 4 or 8)
     bool dense = true;
     int dense_groups_per_cu = 4;
     int dense_waves = 4;
     int dense_small_groups = 0;  // small-grid instance in front (0: off)
-    int dense_large = 1;         // 256-tile instance behind (1 workgroup of 16 waves per CU; 0: off)
+    int dense_large = 1;         // 256-tile instance behind (1 workgroup of 8 waves per CU; 0: off)
     StrokeBuffers stroke;
     AtlasState atlas;
     ~Context();
@@ -160,13 +161,15 @@ struct Context {
 // `unordered` (used for the paths the batched pipeline hands on, under the
 // dense kernels' 1-LSB contract) replaces the sort and the ordered tile pass
 // by window buckets and LDS float-atomic sums.
-int run_plain(Context* ctx, const SegInput& in, OutputDesc& out, hipStream_t stream, bool unordered = false);
-// Persistent work-queue pipeline (one wave per path); paths that do not fit a
-// wave are deferred to run_plain.  waves_per_cu sets the persistent grid,
-// gran the paths taken per queue pop; use_graph replays (reset, kernel) from
-// a captured HIP graph.
-int run_batched(Context* ctx, const SegInput& in, OutputDesc& out, hipStream_t stream, int waves_per_cu, int gran,
-                int tiles_per_chunk, bool use_graph);
+// pass_lines / pass_entries bound a pass below the context's limits (0: no
+// further): a batch over them is split, a single path over them is not refused.
+int run_plain(Context* ctx, const SegInput& in, OutputDesc& out, hipStream_t stream, bool unordered = false,
+              int64_t pass_lines = 0, int64_t pass_entries = 0);
+// The dense kernels over a device queue of paths, then run_plain over the paths
+// they hand on; with the dense kernels off (ctx->dense), run_plain alone.
+// use_graph replays the dense launches from a captured HIP graph where a call
+// repeats the one before.
+int run_batched(Context* ctx, const SegInput& in, OutputDesc& out, hipStream_t stream, bool use_graph);
 // One path by k_single with no host round trip: the output goes where `out`
 // points and the control block (SMALL_CTL_BYTES, reset by the kernel) to
 // `ctl`, both device-visible (pinned host memory mapped into the device's

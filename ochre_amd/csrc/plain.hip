@@ -1963,8 +1963,8 @@ static int run_plain_pass(Context* ctx, const SegInput& in, OutputDesc& out, hip
     if (ht->error & ERR_INPUT) return -1;
     if (ht->error & ERR_FLATTEN) return -5;
     const int64_t L = ht->lines;
-    if (L > ctx->max_lines) {
-        ctx->split_ratio = (double)L / (double)ctx->max_lines;
+    if (L > ctx->pass_lines) {
+        ctx->split_ratio = (double)L / (double)ctx->pass_lines;
         return ST_SPLIT;
     }
 
@@ -2010,8 +2010,8 @@ static int run_plain_pass(Context* ctx, const SegInput& in, OutputDesc& out, hip
     if (ht->error & ERR_FLATTEN) return -5;
     // entries >= runs (every run record is also a sort entry), so below the
     // limit both 32-bit halves of the packed total are exact
-    if (ht->entries > (uint64_t)ctx->max_entries) {
-        ctx->split_ratio = (double)ht->entries / (double)ctx->max_entries;
+    if (ht->entries > (uint64_t)ctx->pass_entries) {
+        ctx->split_ratio = (double)ht->entries / (double)ctx->pass_entries;
         return ST_SPLIT;
     }
     const int64_t R = (int64_t)(uint32_t)ht->dda;
@@ -2294,11 +2294,24 @@ static int check_call_error(Context* ctx, int st, hipStream_t s) {
     return st;
 }
 
-int run_plain(Context* ctx, const SegInput& in, OutputDesc& out, hipStream_t s, bool unordered) {
+int run_plain(Context* ctx, const SegInput& in, OutputDesc& out, hipStream_t s, bool unordered, int64_t pass_lines,
+              int64_t pass_entries) {
     HIPCHK(ctx->call_error.ensure(256));
     if (!ctx->host_pinned) HIPCHK(hipHostMalloc(&ctx->host_pinned, 4096));
     fill<uint32_t>(ctx->call_error.as<uint32_t>(), 1, 0u, s);
-    int st = run_plain_pass(ctx, in, out, s, unordered);
+    // a pass within the asked limits; one path over them, within the context's
+    auto pass = [&](const SegInput& si, OutputDesc& od) {
+        ctx->pass_lines = pass_lines ? std::min(pass_lines, ctx->max_lines) : ctx->max_lines;
+        ctx->pass_entries = pass_entries ? std::min(pass_entries, ctx->max_entries) : ctx->max_entries;
+        const int rc = run_plain_pass(ctx, si, od, s, unordered);
+        if (rc != ST_SPLIT || si.n_paths > 1 ||
+            (ctx->pass_lines == ctx->max_lines && ctx->pass_entries == ctx->max_entries))
+            return rc;
+        ctx->pass_lines = ctx->max_lines;
+        ctx->pass_entries = ctx->max_entries;
+        return run_plain_pass(ctx, si, od, s, unordered);
+    };
+    int st = pass(in, out);
     if (st != ST_SPLIT) return check_call_error(ctx, st, s);
     // Paths are independent Rasterizers: rasterise path ranges one after
     // another, each range's tiles and spans following the previous range's.
@@ -2367,7 +2380,7 @@ int run_plain(Context* ctx, const SegInput& in, OutputDesc& out, hipStream_t s, 
         od.path_span_count = out.path_span_count + p0;
         od.tile_base = out.tile_base + T;
         od.span_base = out.span_base + S;
-        st = run_plain_pass(ctx, si, od, s, unordered);
+        st = pass(si, od);
         if (st == ST_SPLIT) {
             if (n < 2) return -7;
             cut(p0, p1);

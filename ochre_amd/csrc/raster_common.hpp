@@ -303,8 +303,8 @@ __device__ inline bool chain_walk_ok(V2 last, V2 point) {
 // so the increments are the chains' values below 1, plus the last one.  Only
 // for the lines chain_walk_ok covers; returns false, visiting nothing, for
 // the others.
-template <class Tile, class Cross>
-__device__ inline bool line_tiles(V2 last, V2 point, uint32_t& incs, Tile&& tile, Cross&& cross) {
+template <bool INCS, class Tile, class Cross>
+__device__ inline bool line_tiles_of(V2 last, V2 point, uint32_t& incs, Tile&& tile, Cross&& cross) {
     incs = 0;
     if (!chain_walk_ok(last, point)) return false;
     if (veq(point, last)) return true;  // rasterizer.rs:73
@@ -335,13 +335,24 @@ __device__ inline bool line_tiles(V2 last, V2 point, uint32_t& incs, Tile&& tile
             break;
         }
     }
-    uint32_t nx = 0, ny = 0;
-    for (float c = d.col_t1; c < 1.0f; c = fminf(c + d.x_step, 1.0f)) nx++;
-    for (float c = d.row_t1; c < 1.0f; c = fminf(c + d.y_step, 1.0f)) ny++;
-    incs = nx + ny + 1u;
+    if (INCS) {
+        uint32_t nx = 0, ny = 0;
+        for (float c = d.col_t1; c < 1.0f; c = fminf(c + d.x_step, 1.0f)) nx++;
+        for (float c = d.row_t1; c < 1.0f; c = fminf(c + d.y_step, 1.0f)) ny++;
+        incs = nx + ny + 1u;
+    }
     const int32_t ty_end = (int32_t)f2i16(floorf(point.y)) >> 3;  // the snap (rasterizer.rs:118-131)
     if (ty_end != ty) cross((int32_t)f2i16(floorf(point.x)) >> 3, ty_end < ty ? ty_end : ty, (int)(ty_end - ty));
     return true;
+}
+template <class Tile, class Cross>
+__device__ inline bool line_tiles(V2 last, V2 point, uint32_t& incs, Tile&& tile, Cross&& cross) {
+    return line_tiles_of<true>(last, point, incs, tile, cross);
+}
+template <class Tile, class Cross>  // without the increments
+__device__ inline bool line_tiles(V2 last, V2 point, Tile&& tile, Cross&& cross) {
+    uint32_t incs;
+    return line_tiles_of<false>(last, point, incs, tile, cross);
 }
 
 // walk_line's runs and tile-row crossings (for sinks that take no increments)

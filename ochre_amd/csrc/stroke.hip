@@ -426,8 +426,7 @@ int run_stroke(Context* ctx, const SegInput& in, const float* widths, const uint
     int st = stroke_expand(ctx, in, widths, stroke_flags, o, s);
     if (st || in.n_paths <= 0) return st;
     if (batched)
-        return run_batched(ctx, o.in, out, s, ctx->batched_waves_per_cu, ctx->batched_gran, ctx->batched_tc,
-                           ctx->batched_graph);
+        return run_batched(ctx, o.in, out, s, ctx->batched_graph);
     return run_plain(ctx, o.in, out, s);
 }
 

@@ -243,7 +243,7 @@ def build_atlas(ctx: Context, out: DeviceOutput, colors, atlas_size=4096, stream
 def run_to_host(ctx, batch, mode="plain", tile_capacity=None, span_capacity=None):
     """Convenience: upload, rasterise (growing the outputs once if needed)
     and return the per-path host arrays.  Modes: "plain", "batched" (the
-    ordered batched kernel alone), "dense" (the dense kernels in front of it),
+    batched call with the dense kernels off), "dense" (with them on),
     and the same for strokes (batch.widths): "stroke_plain",
     "stroke_batched", "stroke_dense", and for draw lists (batch.strokes,
     batch.widths): "draw_plain", "draw_batched", "draw_dense".  The
@@ -323,7 +323,7 @@ def set_dense_small(ctx: Context, groups_per_cu=0):
 
 def set_dense_params(ctx: Context, enabled=True, groups_per_cu=4, waves_per_group=4):
     """The dense single-walk kernel (order-independent f32 sums, alpha within
-    1 LSB of the ordered result) in front of the ordered kernel."""
+    1 LSB of the ordered result); off: the plain pipeline's ordered sums."""
     _lib.check(ctx.lib.ochre_context_set_dense_params(ctx.h, 1 if enabled else 0, groups_per_cu, waves_per_group),
                "set_dense_params")
 
