@@ -42,3 +42,18 @@ def test_dense_hands_on_large_paths(gpu_ctx, n_large):
         assert np.array_equal(want[k], got[k]), k
     d = np.abs(want[1].astype(np.int16) - got[1].astype(np.int16))
     assert int(d.max()) <= 1 and float((d != 0).mean()) < 1e-3
+
+
+@pytest.mark.parametrize("n_first,n_rest,spread", [(2046, 0, 60.0), (2047, 1, 60.0), (3000, 500, 60.0), (2100, 40, 600.0),
+                                                   (3000, 3000, 160.0)])
+def test_dense_paths_of_many_points(gpu_ctx, n_first, n_rest, spread):
+    """Paths over the point count that is tested early: those that fit an instance, and those that
+    only their last points put over it."""
+    import oracle_ref
+    from parity import compare
+    rng = np.random.default_rng(n_first + n_rest)
+    p = np.concatenate([rng.random((n_first, 2)) * 40.0, rng.random((n_rest, 2)) * spread]).astype(np.float32)
+    verbs = [W.MOVE] + [W.LINE] * (len(p) - 1) + [W.CLOSE]
+    b = W.concat([W.from_paths([(verbs, p)], np.array([1, 0, 0, 1, 3.25, 7.5], np.float32)), W.glyph_run(5, seed=83)])
+    stats = compare(oracle_ref.run_batch(b), run_to_host(gpu_ctx, b, "dense", 20000, 20000), max_lsb=1)
+    assert stats["bit_exact_fraction"] >= 0.98  # sums of thousands of increments in arrival order
