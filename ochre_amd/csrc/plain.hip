@@ -1495,8 +1495,8 @@ constexpr int RT_ROWS = TILE / RT_NW;  // pixel rows whose carry each wave takes
 static_assert(RT_ROWS * RT_NW == TILE && RT_ROWS <= 2, "the carry takes one or two pixel rows per wave");
 constexpr int RT_U = 2;  // entries per thread whose loads are issued together
 
-// The window's per-pixel sums are fixed point in f64 slots (fx_of: units of
-// 2^-30, integer-valued): the sums of the increments (|area|, |height| <= 1 +
+// The window's per-pixel sums are fixed point (fx_of: 64-bit integers in units of
+// 2^-30): the sums of the increments (|area|, |height| <= 1 +
 // a few ulps, each truncated at 2^-30) are then exact, so that the decoded f32
 // sum is the correctly rounded sum of the increments, independent of arrival
 // order.  A window of a full-range path (coordinates that may be huge or
@@ -1515,54 +1515,9 @@ struct RowLds {
     uint32_t nt, ns, nocc;
 };
 
-// The increments of a run from the DDA state at its first one (p0: that
-// increment's start point), into the window's LDS sums; CARRY: every active
-// lane's line is finite, so each increment's start point is the previous one's
-// end point (see dda_increment_carried).
-template <bool EMIT, bool CARRY>
-__device__ inline void rt_replay_steps(RowLds<EMIT>& s, Dda& d, V2 p0, bool finite, uint32_t x, bool fx,
-                                       Counters* cnt) {
-    // the pixel within the run's tile: the run ends when it leaves 0..7 on
-    // either axis (or the line ends)
-    uint32_t lx = (uint32_t)(d.x & 7), ly = (uint32_t)(d.y & 7);
-    const uint32_t xb = x * (uint32_t)UWS;
-    const uint32_t lxd = (uint32_t)(int32_t)d.x_dir, lyd = (uint32_t)(int32_t)d.y_dir;
-    bool ended = false;
-    for (int k = 0; k < 16; k++) {
-        float area, height;
-        dda_increment_carried(d, p0, CARRY || finite, area, height);
-        const uint32_t px = xb + ((ly << 3) | lx);
-        if (fx) {
-            atomicAdd(reinterpret_cast<double*>(&s.acc_a[px]), fx_of(area));
-            atomicAdd(reinterpret_cast<double*>(&s.acc_h[px]), fx_of(height));
-        } else {
-            atomicAdd(reinterpret_cast<float*>(&s.acc_a[px]), area);
-            atomicAdd(reinterpret_cast<float*>(&s.acc_h[px]), height);
-        }
-        // dda_step, with the in-tile pixel moved alongside
-        float c;
-        if (d.row_t1 < d.col_t1) {
-            c = d.row_t1;
-            d.row_t1 = fminf(d.row_t1 + d.y_step, 1.0f);
-            d.y = wrap16(d.y + d.y_dir);
-            ly += lyd;
-        } else {
-            c = d.col_t1;
-            d.col_t1 = fminf(d.col_t1 + d.x_step, 1.0f);
-            d.x = wrap16(d.x + d.x_dir);
-            lx += lxd;
-        }
-        d.t0 = c;
-        if (c == 1.0f || (lx | ly) > 7u) {
-            ended = true;
-            break;
-        }
-    }
-    if (!ended) atomicOr(&cnt->error, (uint32_t)ERR_REPLAY);
-}
-
-// Replays a run (x: its tile within the window) into the window's LDS sums
-// (fixed-point or float atomics, arrival order).
+// Replays a run (x: its tile within the window) into the window's LDS sums, in
+// arrival order: fixed point where fx, else float atomics.  In an fx window every
+// path is within +-HUGE_COORD, so FastWalk covers its lines.
 template <bool EMIT>
 __device__ inline void rt_replay_run(RowLds<EMIT>& s, uint32_t x, const RunRec& rr, const float4& L, bool fx,
                                      Counters* cnt) {
@@ -1579,11 +1534,42 @@ __device__ inline void rt_replay_run(RowLds<EMIT>& s, uint32_t x, const RunRec& 
         d.t0 = 0.0f;
         dda_step(d);
     }
+    V2 p0 = dda_point(d, d.t0);
+    // the pixel within the run's tile as two nibbles, y above x: leaving 0..7 on
+    // either axis sets a nibble's top bit
+    uint32_t at = (uint32_t)(((d.y & 7) << 4) | (d.x & 7));
+    const uint32_t xd = (uint32_t)(int32_t)d.x_dir, yd = (uint32_t)((int32_t)d.y_dir * 16);
+    const uint32_t xb = x * (uint32_t)UWS;
+    if (fx) {
+        FastWalk w;
+        w.init(d, p0);
+        for (;;) {  // (at most 15 steps: each moves one pixel on, the same way along its axis)
+            float area, height;
+            bool y;
+            const bool end = w.step(area, height, y);
+            const uint32_t px = xb + at - ((at >> 4) << 3);
+            atomicAdd(reinterpret_cast<unsigned long long*>(&s.acc_a[px]), fx_of(area));
+            atomicAdd(reinterpret_cast<unsigned long long*>(&s.acc_h[px]), fx_of(height));
+            at += y ? yd : xd;
+            if (end || (at & 0x88u)) break;
+        }
+        return;
+    }
     const bool finite = line_finite(last, point);
-    const V2 p0 = dda_point(d, d.t0);
-    // a wave-uniform choice: the start-point recomputation only where a line needs it
-    if (__ballot(!finite) == 0) rt_replay_steps<EMIT, true>(s, d, p0, finite, x, fx, cnt);
-    else rt_replay_steps<EMIT, false>(s, d, p0, finite, x, fx, cnt);
+    bool ended = false;
+    for (int k = 0; k < 16; k++) {
+        float area, height;
+        dda_increment_carried(d, p0, finite, area, height);
+        const uint32_t px = xb + at - ((at >> 4) << 3);
+        atomicAdd(reinterpret_cast<float*>(&s.acc_a[px]), area);
+        atomicAdd(reinterpret_cast<float*>(&s.acc_h[px]), height);
+        at += d.row_t1 < d.col_t1 ? yd : xd;
+        if (dda_step(d) || (at & 0x88u)) {
+            ended = true;
+            break;
+        }
+    }
+    if (!ended) atomicOr(&cnt->error, (uint32_t)ERR_REPLAY);
 }
 
 // RT_U entries per thread of a window (entries e0 + u * RT_NT), with their
@@ -1784,7 +1770,7 @@ __global__ __launch_bounds__(RT_NT) void k_row_tiles(RowTileArgs a) {
                         float* fh = reinterpret_cast<float*>(s.acc_h);  // the slots' low words
 #pragma unroll
                         for (int k = 0; k < 8; k++) {
-                            const float h = fx ? fx_to_f(reinterpret_cast<const double*>(s.acc_h)[base + k])
+                            const float h = fx ? fx_to_f(s.acc_h[base + k])
                                                : fh[2 * (base + k)];
                             fh[2 * (base + k)] = tot;
                             tot += h;
@@ -1811,7 +1797,7 @@ __global__ __launch_bounds__(RT_NT) void k_row_tiles(RowTileArgs a) {
                     const float* fa = reinterpret_cast<const float*>(s.acc_a);
 #pragma unroll
                     for (int k = 0; k < 4; k++) {
-                        const float av = fx ? fx_to_f(reinterpret_cast<const double*>(s.acc_a)[base + k])
+                        const float av = fx ? fx_to_f(s.acc_a[base + k])
                                             : fa[2 * (base + k)];
                         const float v = (cin + fh[2 * (base + k)]) + av;
                         word |= (uint32_t)fminf(fabsf(v) * 256.0f, 255.0f) << (8 * k);

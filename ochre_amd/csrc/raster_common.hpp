@@ -168,19 +168,18 @@ struct BoxAcc {
     }
 };
 
-// Per-pixel sums of the unordered tile stage in fixed point, units of 2^-30,
-// held as integer-valued f64: an increment's |area|, |height| <= 1 plus a few
-// ulps for lines with finite coordinates within +-30000, so the sums of 2^22 of
-// them stay below 2^53 units, where every f64 sum of integers is exact; the
-// sum is then independent of arrival order, and the decoded f32 value is the
-// correctly rounded sum of the increments (each truncated at 2^-30).  The
-// conversion is three f64 operations (f32 to f64, scale, truncate), where a
-// 64-bit integer one needs ten.
-constexpr double FX_SCALE = 1073741824.0;       // 2^30
+// Per-pixel sums of the unordered tile stage in fixed point, 64-bit integers in
+// units of 2^-30: an increment's |area|, |height| <= 1 plus the rounding of
+// coordinates within +-30000 (below 2), so it converts through 32 bits (a
+// multiplication, a truncation and the sign: half the cost of the same in f64), and
+// the sums of 2^22 of them stay below 2^53 units; the sum is then independent of
+// arrival order, and the decoded f32 value is the correctly rounded sum of the
+// increments (each truncated at 2^-30).
+constexpr float FX_SCALE = 1073741824.0f;           // 2^30
 constexpr double FX_UNIT = 9.313225746154785e-10;  // 2^-30
 
-__device__ inline double fx_of(float v) { return trunc((double)v * FX_SCALE); }
-__device__ inline float fx_to_f(double q) { return (float)(q * FX_UNIT); }
+__device__ inline unsigned long long fx_of(float v) { return (unsigned long long)(long long)(int32_t)(v * FX_SCALE); }
+__device__ inline float fx_to_f(long long q) { return (float)((double)q * FX_UNIT); }
 
 // ------------------------------------------------------ (b) DDA binning
 //
