@@ -591,13 +591,22 @@ int run_batched(Context* ctx, const SegInput& in, OutputDesc& out, hipStream_t s
     const int n_small = cus * std::max(0, ctx->dense_small_groups);
     const int n_large = ctx->dense_large ? cus : 0;
     // The dense instances run one after another, each over the paths the one
-    // before handed on: [small grids, 32 tiles] -> 64 tiles -> [256 tiles]; what is
+    // before handed on: [small grids, 32 tiles] -> 64 tiles -> [256 tiles], or the
+    // 256-tile one alone over few paths; what is
     // left goes to the plain pipeline.
-    enum { D_SMALL, D_MAIN, D_LARGE };
+    enum { D_SMALL, D_MAIN, D_LARGE, D_FEW };
     int stages[3], n_stages = 0;
-    if (n_small) stages[n_stages++] = D_SMALL;
-    stages[n_stages++] = D_MAIN;
-    if (n_large) stages[n_stages++] = D_LARGE;
+    // With a CU for every path, each gets 16 waves of the 256-tile instance and one
+    // launch: a path's latency is all there is (61 glyphs of 12-48 px 81 -> 68 us a
+    // call, 256 of them 91 -> 71, 61 of 60-120 px 264 -> 238; at 512 paths, two to a
+    // CU one after the other, 95 -> 108).
+    if (n_large && NP <= cus) {
+        stages[n_stages++] = D_FEW;
+    } else {
+        if (n_small) stages[n_stages++] = D_SMALL;
+        stages[n_stages++] = D_MAIN;
+        if (n_large) stages[n_stages++] = D_LARGE;
+    }
     HIPCHK_RET(B->dense_ids.ensure((size_t)NP * 4));
     if (n_stages > 1) HIPCHK_RET(B->dense_ids2.ensure((size_t)NP * 4));
     if (n_stages > 2) HIPCHK_RET(B->dense_ids3.ensure((size_t)NP * 4));
@@ -621,7 +630,10 @@ int run_batched(Context* ctx, const SegInput& in, OutputDesc& out, hipStream_t s
         if (ev) (void)hipEventRecord(ctx->ev[0], st);
         for (int i = 0; i < n_stages; i++) {
             const FusedIn& f = fin[i];
-            if (stages[i] == D_SMALL)
+            if (stages[i] == D_FEW)
+                hipLaunchKernelGGL((k_dense<16, 256>), dim3((unsigned)NP), dim3(16 * WAVE), 0, st, f, fo, ctl,
+                                   queues[i], lists[i], counts[i]);
+            else if (stages[i] == D_SMALL)
                 hipLaunchKernelGGL((k_dense<2, 32>), dim3(n_small), dim3(2 * WAVE), 0, st, f, fo, ctl, queues[i],
                                    lists[i], counts[i]);
             else if (stages[i] == D_LARGE)
@@ -656,7 +668,7 @@ int run_batched(Context* ctx, const SegInput& in, OutputDesc& out, hipStream_t s
         put(&dnw, 4);
         put(&n_groups, 4);
         put(&n_small, 4);
-        put(&n_large, 4);
+        put(&n_large, 4);  // (and the path count, in fi: they decide the stages)
         replay = B->exec && key == B->graph_key;
         if (!replay && key == B->last_key) {
             if (B->exec) (void)hipGraphExecDestroy(B->exec);

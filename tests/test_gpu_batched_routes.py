@@ -57,3 +57,13 @@ def test_dense_paths_of_many_points(gpu_ctx, n_first, n_rest, spread):
     b = W.concat([W.from_paths([(verbs, p)], np.array([1, 0, 0, 1, 3.25, 7.5], np.float32)), W.glyph_run(5, seed=83)])
     stats = compare(oracle_ref.run_batch(b), run_to_host(gpu_ctx, b, "dense", 20000, 20000), max_lsb=1)
     assert stats["bit_exact_fraction"] >= 0.98  # sums of thousands of increments in arrival order
+
+
+@pytest.mark.parametrize("n", [1, 2, 255, 256, 257])
+def test_dense_few_paths(gpu_ctx, n):
+    """Path counts around one per compute unit: sets exact, alpha within 1 LSB of the oracle's."""
+    import oracle_ref
+    from parity import compare
+    b = W.glyph_run(n, seed=90 + n, smin=12.0, smax=110.0)
+    stats = compare(oracle_ref.run_batch(b), run_to_host(gpu_ctx, b, "dense", n * 300 + 100, n * 300 + 100), max_lsb=1)
+    assert stats["bit_exact_fraction"] >= 0.999
