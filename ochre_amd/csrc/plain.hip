@@ -2017,9 +2017,11 @@ static int run_plain_pass(Context* ctx, const SegInput& in, OutputDesc& out, hip
     HIPCHK(ctx->vals[0].ensure(std::max<int64_t>(R, 1) * 4));
     HIPCHK(ctx->vals[1].ensure(std::max<int64_t>(R, 1) * 4));
     HIPCHK(ctx->records.ensure(std::max<int64_t>(RUNS, 1) * sizeof(RunRec)));
-    const uint32_t rs_blocks = (uint32_t)std::max<int64_t>(1, (R + RS_TILE - 1) / RS_TILE);
-    HIPCHK(ctx->rs_counts.ensure((size_t)rs_blocks * 256 * 4));
-    HIPCHK(ensure_scan_capacity(ctx, std::max<int64_t>({R, (int64_t)rs_blocks * 256, ROWS, 1})));
+    const int rs_bits = rs_digit_bits((int)kbits);
+    const int64_t rs_tile = (int64_t)RS_NT * rs_items(R);
+    const uint32_t rs_blocks = (uint32_t)std::max<int64_t>(1, (R + rs_tile - 1) / rs_tile);
+    if (!unordered) HIPCHK(ctx->rs_counts.ensure(((size_t)rs_blocks << rs_bits) * 4));
+    HIPCHK(ensure_scan_capacity(ctx, std::max<int64_t>({unordered ? 1 : (int64_t)rs_blocks << rs_bits, ROWS, 1})));
     da.xbits = xbits;
     da.keys = ctx->keys[0].as<uint32_t>();
     da.vals = ctx->vals[0].as<uint32_t>();
@@ -2141,19 +2143,30 @@ static int run_plain_pass(Context* ctx, const SegInput& in, OutputDesc& out, hip
         return 0;
     }
     int cur = 0;
-    const int passes = (int)((kbits + 7) / 8);
     uint32_t* rsc = ctx->rs_counts.as<uint32_t>();
-    for (int pass = 0; pass < passes && R > 0; pass++) {
-        int shift = pass * 8;
-        hipLaunchKernelGGL(k_rs_count, dim3(rs_blocks), dim3(RS_NT), 0, s, ctx->keys[cur].as<uint32_t>(), R, shift,
-                           rsc, rs_blocks);
-        HIPCHK(launch_scan<uint32_t>(ctx, (int64_t)rs_blocks * 256, LoadU32{rsc}, StoreU32{rsc}, OpAdd(), 0u,
-                                     (uint32_t*)nullptr, s));
-        // values are the entry payloads (run index, or crossing sign with bit 31)
-        hipLaunchKernelGGL(k_rs_scatter, dim3(rs_blocks), dim3(RS_NT), 0, s, ctx->keys[cur].as<uint32_t>(),
-                           ctx->vals[cur].as<uint32_t>(), R, shift, rsc, rs_blocks,
-                           ctx->keys[cur ^ 1].as<uint32_t>(), ctx->vals[cur ^ 1].as<uint32_t>());
+    auto sort_pass = [&](auto bits, auto items, int shift) -> hipError_t {
+        constexpr int B = decltype(bits)::value, I = decltype(items)::value;
+        uint32_t *kin = ctx->keys[cur].as<uint32_t>(), *vin = ctx->vals[cur].as<uint32_t>();
+        hipLaunchKernelGGL((k_rs_count<B, I>), dim3(rs_blocks), dim3(RS_NT), 0, s, kin, R, shift, rsc, rs_blocks);
+        const hipError_t e = launch_scan<uint32_t>(ctx, (int64_t)rs_blocks << B, LoadU32{rsc}, StoreU32{rsc}, OpAdd(),
+                                                   0u, (uint32_t*)nullptr, s);
+        if (e != hipSuccess) return e;
+        // values are the entry payloads (a run, or crossing sign with bit 31)
+        hipLaunchKernelGGL((k_rs_scatter<B, I>), dim3(rs_blocks), dim3(RS_NT), 0, s, kin, vin, R, shift, rsc,
+                           rs_blocks, ctx->keys[cur ^ 1].as<uint32_t>(), ctx->vals[cur ^ 1].as<uint32_t>());
         cur ^= 1;
+        return hipSuccess;
+    };
+    using B8 = std::integral_constant<int, 8>;
+    using B10 = std::integral_constant<int, 10>;
+    using Large = std::integral_constant<int, RS_ITEMS_LARGE>;
+    using Small = std::integral_constant<int, RS_ITEMS_SMALL>;
+    const bool rs_small = rs_items(R) == RS_ITEMS_SMALL;
+    for (int shift = 0; shift < (int)kbits && R > 0; shift += rs_bits) {
+        if (rs_bits == 10)
+            HIPCHK(rs_small ? sort_pass(B10(), Small(), shift) : sort_pass(B10(), Large(), shift));
+        else
+            HIPCHK(rs_small ? sort_pass(B8(), Small(), shift) : sort_pass(B8(), Large(), shift));
     }
     const uint32_t* skeys = ctx->keys[cur].as<uint32_t>();
     const uint32_t* svals = ctx->vals[cur].as<uint32_t>();

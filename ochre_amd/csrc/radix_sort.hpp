@@ -1,5 +1,5 @@
-// Stable LSD radix sort of (u32 key, u32 value) pairs, 8-bit digits, for
-// wave64.  Each pass: per-block digit counts -> device scan (digit-major) ->
+// Stable LSD radix sort of (u32 key, u32 value) pairs, digits of 8 or 10 bits,
+// for wave64.  Each pass: per-block digit counts -> device scan (digit-major) ->
 // scatter with stable block-local ranks computed by per-wave ballot matching.
 // Stability is what makes equal tile keys keep the emission order that the
 // per-pixel f32 sums depend on.
@@ -9,11 +9,18 @@
 
 namespace ochre {
 
-constexpr int RS_NT = 256;                 // threads per block
-constexpr int RS_ITEMS = 16;               // keys per thread
-constexpr int RS_TILE = RS_NT * RS_ITEMS;  // 4096 keys per block
+constexpr int RS_NT = 256;  // threads per block
 constexpr int RS_WAVES = RS_NT / WAVE;
-constexpr int RS_WAVE_ITEMS = RS_TILE / RS_WAVES;  // 1024
+// Keys per thread: 16, or 4 for small inputs, whose blocks would otherwise be too
+// few to reach every CU (a plain call of 61 glyphs, 15,000 keys: 270 us with 4,
+// 278 with 16; 150,000 keys 308 / 326, 300,000 348 / 348, 600,000 450 / 416).
+constexpr int RS_ITEMS_LARGE = 16, RS_ITEMS_SMALL = 4;
+constexpr int64_t RS_SMALL = (int64_t)1 << 18;  // keys up to which a block takes 4 per thread
+inline int rs_items(int64_t n) { return n <= RS_SMALL ? RS_ITEMS_SMALL : RS_ITEMS_LARGE; }
+// Digit width: 10 bits where that saves a pass over 8 (a plain call of 2,500 glyphs,
+// 18-bit keys: 438 -> 417 us, 10,000 glyphs, 20 bits: 838 -> 827; k_rs_scatter 50 us
+// a pass either way on 2.4 million keys).
+inline int rs_digit_bits(int key_bits) { return (key_bits + 9) / 10 < (key_bits + 7) / 8 ? 10 : 8; }
 
 __device__ inline uint64_t lanemask_lt() {
     const int lane = lane_id();
@@ -21,24 +28,26 @@ __device__ inline uint64_t lanemask_lt() {
 }
 
 // counts[digit * nblocks + block]
+template <int BITS, int ITEMS>
 __global__ __launch_bounds__(RS_NT) void k_rs_count(const uint32_t* __restrict__ keys, int64_t n, int shift,
                                                     uint32_t* __restrict__ counts, uint32_t nblocks) {
-    __shared__ uint32_t hist[RS_WAVES][256];
+    constexpr int DIGITS = 1 << BITS;
+    __shared__ uint32_t hist[RS_WAVES][DIGITS];
     const int tid = threadIdx.x;
     const int wid = tid / WAVE;
-    for (int i = tid; i < RS_WAVES * 256; i += RS_NT) (&hist[0][0])[i] = 0;
+    for (int i = tid; i < RS_WAVES * DIGITS; i += RS_NT) (&hist[0][0])[i] = 0;
     __syncthreads();
-    const int64_t base = (int64_t)blockIdx.x * RS_TILE;
+    const int64_t base = (int64_t)blockIdx.x * (RS_NT * ITEMS);
 #pragma unroll
-    for (int j = 0; j < RS_ITEMS; j++) {
+    for (int j = 0; j < ITEMS; j++) {
         int64_t i = base + (int64_t)j * RS_NT + tid;
         if (i < n) {
-            uint32_t d = (keys[i] >> shift) & 255u;
+            uint32_t d = (keys[i] >> shift) & (DIGITS - 1u);
             atomicAdd(&hist[wid][d], 1u);
         }
     }
     __syncthreads();
-    for (int d = tid; d < 256; d += RS_NT) {
+    for (int d = tid; d < DIGITS; d += RS_NT) {
         uint32_t s = 0;
 #pragma unroll
         for (int w = 0; w < RS_WAVES; w++) s += hist[w][d];
@@ -47,93 +56,103 @@ __global__ __launch_bounds__(RS_NT) void k_rs_count(const uint32_t* __restrict__
 }
 
 // Scatter.  offsets[digit * nblocks + block] = exclusive global start.
-// vals_in == nullptr means the identity permutation (value = index).
-// The block's keys are first placed in LDS in digit order (block-local stable
+// The block's pairs are first placed in LDS in digit order (block-local stable
 // positions: digit start + the wave's offset in the digit + the rank within
 // the wave), then written out in that order, so that consecutive threads
-// store consecutive addresses of one digit's run; the values follow through
-// the same positions.
-static_assert(RS_NT == 256, "the scatter takes one digit per thread");
-
+// store consecutive addresses of one digit's run.
+template <int BITS, int ITEMS>
 struct RsScatterLds {
-    uint32_t cnt[RS_WAVES][256];  // per wave and digit: count, then the wave's start within the digit
-    uint32_t dstart[256];         // the digit's first position in the block
-    uint32_t goff[256];           // the digit's global start for this block
-    uint32_t buf[RS_TILE];        // keys, then values, in digit order
-    uint8_t dig[RS_TILE];         // the digit at each position
+    static constexpr int DIGITS = 1 << BITS, TILE_KEYS = RS_NT * ITEMS;
+    uint16_t cnt[RS_WAVES][DIGITS];  // per wave and digit: count, then the wave's start within the digit
+    uint16_t dstart[DIGITS];         // the digit's first position in the block
+    uint32_t goff[DIGITS];           // the digit's global start for this block
+    uint32_t wtot[RS_WAVES];
+    uint32_t buf[TILE_KEYS];  // keys, then values, in digit order
+    uint16_t dig[TILE_KEYS];  // the digit at each position
 };
 
+template <int BITS, int ITEMS>
 __global__ __launch_bounds__(RS_NT, 4) void k_rs_scatter(const uint32_t* __restrict__ keys_in,
                                                       const uint32_t* __restrict__ vals_in, int64_t n, int shift,
                                                       const uint32_t* __restrict__ offsets, uint32_t nblocks,
                                                       uint32_t* __restrict__ keys_out,
                                                       uint32_t* __restrict__ vals_out) {
-    __shared__ RsScatterLds s;
+    using Lds = RsScatterLds<BITS, ITEMS>;
+    constexpr int DIGITS = Lds::DIGITS, PER = DIGITS / RS_NT;  // consecutive digits per thread
+    __shared__ Lds s;
     const int tid = threadIdx.x;
     const int wid = tid / WAVE;
     const int lane = lane_id();
-    for (int i = tid; i < RS_WAVES * 256; i += RS_NT) (&s.cnt[0][0])[i] = 0;
-    for (int d = tid; d < 256; d += RS_NT) s.goff[d] = offsets[(int64_t)d * nblocks + blockIdx.x];
+    for (int i = tid; i < RS_WAVES * DIGITS; i += RS_NT) (&s.cnt[0][0])[i] = 0;
+    for (int d = tid; d < DIGITS; d += RS_NT) s.goff[d] = offsets[(int64_t)d * nblocks + blockIdx.x];
     __syncthreads();
     const uint64_t lt = lanemask_lt();
-    // Items of wave w: base + w*1024 + j*64 + lane, so (j, lane) order is index order.
-    const int64_t bbase = (int64_t)blockIdx.x * RS_TILE;
-    const int64_t wbase = bbase + (int64_t)wid * RS_WAVE_ITEMS;
-    const int nb = (int)(n - bbase < (int64_t)RS_TILE ? n - bbase : (int64_t)RS_TILE);  // items in this block
-    uint32_t key[RS_ITEMS];
-    uint32_t rank[RS_ITEMS];
+    // Items of wave w: base + w*64*ITEMS + j*64 + lane, so (j, lane) order is index order.
+    const int64_t bbase = (int64_t)blockIdx.x * Lds::TILE_KEYS;
+    const int64_t wbase = bbase + (int64_t)wid * (WAVE * ITEMS);
+    const int nb = (int)(n - bbase < (int64_t)Lds::TILE_KEYS ? n - bbase : (int64_t)Lds::TILE_KEYS);  // items in this block
+    uint32_t key[ITEMS], val[ITEMS];
+    uint32_t rank[ITEMS];
 #pragma unroll
-    for (int j = 0; j < RS_ITEMS; j++) {
+    for (int j = 0; j < ITEMS; j++) {
         int64_t i = wbase + (int64_t)j * WAVE + lane;
-        bool valid = i < n;
-        uint32_t k = valid ? keys_in[i] : 0u;
-        key[j] = k;
-        uint32_t d = (k >> shift) & 255u;
+        key[j] = i < n ? keys_in[i] : 0u;
+        val[j] = i < n ? vals_in[i] : 0u;
+    }
+#pragma unroll
+    for (int j = 0; j < ITEMS; j++) {
+        bool valid = wbase + (int64_t)j * WAVE + lane < n;
+        uint32_t d = (key[j] >> shift) & (DIGITS - 1u);
         uint64_t match = __ballot(valid);
 #pragma unroll
-        for (int b = 0; b < 8; b++) {
+        for (int b = 0; b < BITS; b++) {
             uint64_t m = __ballot((d >> b) & 1u);
             match &= ((d >> b) & 1u) ? m : ~m;
         }
         uint32_t prior = valid ? s.cnt[wid][d] : 0u;
         rank[j] = prior + (uint32_t)__popcll(match & lt);
         // The lowest lane of each match group advances the wave-private counter.
-        if (valid && (match & lt) == 0) s.cnt[wid][d] = prior + (uint32_t)__popcll(match);
+        if (valid && (match & lt) == 0) s.cnt[wid][d] = (uint16_t)(prior + (uint32_t)__popcll(match));
     }
     __syncthreads();
-    // per digit: the waves' starts within the digit, and the digit's total
-    uint32_t tot = 0;
+    // per digit: the waves' starts within the digit, and the digit's total; the
+    // digits' starts in the block by a scan of the totals
     {
-        const int d = tid;  // RS_NT == 256: one thread per digit
+        uint32_t tot[PER], sum = 0;
 #pragma unroll
-        for (int w = 0; w < RS_WAVES; w++) {
-            const uint32_t c = s.cnt[w][d];
-            s.cnt[w][d] = tot;
-            tot += c;
+        for (int k = 0; k < PER; k++) {
+            const int d = tid * PER + k;
+            tot[k] = 0;
+#pragma unroll
+            for (int w = 0; w < RS_WAVES; w++) {
+                const uint32_t c = s.cnt[w][d];
+                s.cnt[w][d] = (uint16_t)tot[k];
+                tot[k] += c;
+            }
+            sum += tot[k];
         }
-    }
-    // the digits' starts in the block: a block scan of the totals
-    {
-        const uint32_t incl = wave_incl_scan(tot, OpAdd());
-        if (lane == WAVE - 1) s.dstart[wid] = incl;  // wave totals (dstart reused below)
+        const uint32_t incl = wave_incl_scan(sum, OpAdd());
+        if (lane == WAVE - 1) s.wtot[wid] = incl;
         __syncthreads();
-        uint32_t before = 0;
+        uint32_t at = incl - sum;
 #pragma unroll
         for (int w = 0; w < RS_WAVES; w++)
-            if (w < wid) before += s.dstart[w];
-        __syncthreads();
-        s.dstart[tid] = before + incl - tot;
+            if (w < wid) at += s.wtot[w];
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            s.dstart[tid * PER + k] = (uint16_t)at;
+            at += tot[k];
+        }
     }
     __syncthreads();
     // rank[j] becomes the item's position in the block
 #pragma unroll
-    for (int j = 0; j < RS_ITEMS; j++) {
-        int64_t i = wbase + (int64_t)j * WAVE + lane;
-        if (i < n) {
-            const uint32_t d = (key[j] >> shift) & 255u;
-            rank[j] += s.dstart[d] + s.cnt[wid][d];
+    for (int j = 0; j < ITEMS; j++) {
+        if (wbase + (int64_t)j * WAVE + lane < n) {
+            const uint32_t d = (key[j] >> shift) & (DIGITS - 1u);
+            rank[j] += (uint32_t)s.dstart[d] + s.cnt[wid][d];
             s.buf[rank[j]] = key[j];
-            s.dig[rank[j]] = (uint8_t)d;
+            s.dig[rank[j]] = (uint16_t)d;
         }
     }
     __syncthreads();
@@ -143,10 +162,8 @@ __global__ __launch_bounds__(RS_NT, 4) void k_rs_scatter(const uint32_t* __restr
     }
     __syncthreads();
 #pragma unroll
-    for (int j = 0; j < RS_ITEMS; j++) {
-        int64_t i = wbase + (int64_t)j * WAVE + lane;
-        if (i < n) s.buf[rank[j]] = vals_in ? vals_in[i] : (uint32_t)i;
-    }
+    for (int j = 0; j < ITEMS; j++)
+        if (wbase + (int64_t)j * WAVE + lane < n) s.buf[rank[j]] = val[j];
     __syncthreads();
     for (int i = tid; i < nb; i += RS_NT) {
         const uint32_t d = s.dig[i];
