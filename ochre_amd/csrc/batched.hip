@@ -99,7 +99,10 @@ template <int TC>
 struct LdsState {
     uint32_t occ[F_GRID];
     uint32_t row_rank[F_GRID + 1];
-    uint32_t chunk_tile[TC];
+    struct {  // lines queued for a walk of the adjoint
+        float4 line[2 * WAVE];
+        uint16_t id[2 * WAVE];
+    } q;
     // tsign is dead once spans are written; the accumulators live after that
     union {
         int32_t tsign[F_GRID * F_GRID];
@@ -121,44 +124,6 @@ template <class S>
 __device__ inline uint32_t tile_rank(const S& s, int tx, int ty) {
     return s.row_rank[ty] + (uint32_t)__popc(s.occ[ty] & ((1u << tx) - 1u));
 }
-
-// Two 64-line windows of the line list held in registers (lane i holds lines
-// base + i and base + 64 + i), so refilling lanes read a line with __shfl
-// instead of a dependent global load.
-struct LineWindow {
-    float4 w0, w1;
-    uint32_t base;
-    __device__ void load(const float4* lines, uint32_t L, uint32_t b, int lane) {
-        base = b;
-        const uint32_t i0 = b + lane, i1 = b + 64 + lane;
-        w0 = i0 < L ? lines[i0] : make_float4(0, 0, 0, 0);
-        w1 = i1 < L ? lines[i1] : make_float4(0, 0, 0, 0);
-    }
-    // Fetches line `my` (must be in [base, base + 128)) for every lane.
-    __device__ float4 get(uint32_t my) const {
-        const uint32_t src = my - base;
-        const int sl = (int)(src & 63u);
-        float4 a, b;
-        a.x = __shfl(w0.x, sl, WAVE);
-        a.y = __shfl(w0.y, sl, WAVE);
-        a.z = __shfl(w0.z, sl, WAVE);
-        a.w = __shfl(w0.w, sl, WAVE);
-        b.x = __shfl(w1.x, sl, WAVE);
-        b.y = __shfl(w1.y, sl, WAVE);
-        b.z = __shfl(w1.z, sl, WAVE);
-        b.w = __shfl(w1.w, sl, WAVE);
-        return src < 64 ? a : b;
-    }
-    // Slides by 64 once `next` has passed the first window.
-    __device__ void advance(const float4* lines, uint32_t L, uint32_t next, int lane) {
-        if (next >= base + 64) {
-            w0 = w1;
-            base += 64;
-            const uint32_t i1 = base + 64 + lane;
-            w1 = i1 < L ? lines[i1] : make_float4(0, 0, 0, 0);
-        }
-    }
-};
 
 // Adjoint inputs/outputs (see adjoint.hip).  The target of path p is its
 // tiles [tt_start[p], +tt_count[p]) (row-major, 64 f32 coverages each) and

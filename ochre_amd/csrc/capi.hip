@@ -356,9 +356,9 @@ int ochre_coverage_adjoint(ochre_context* ctx, const ochre_path_batch* in, const
     t.span_count = target->span_count;
     t.span_xy = target->span_xy;
     t.span_w = target->span_width;
-    // The adjoint's own launch shape: on 4,096 16-cubic glyphs 32-tile chunks, a path per pop and
-    // 8 or more waves per CU measured 1.58-1.61 ms, 16-tile chunks 2.37-2.42,
-    // one wave per CU 6.6-9.8 ms.
+    // The adjoint's own launch shape, on 4,096 paths of 16 cubics: 32-tile chunks
+    // (20 KB of LDS, 8 waves per CU) 918 us, 16-tile chunks with 16 waves per CU
+    // 1,149 (twice the walks), one wave per CU 6.6-9.8 ms.
     return run_adjoint(&ctx->c, si, t, loss, d_points, d_transforms, reinterpret_cast<hipStream_t>(stream), 8, 1,
                        32);
 }
