@@ -109,7 +109,6 @@ struct LdsState {
         struct {
             float acc_a[TC * F_TSTRIDE];
             float acc_h[TC * F_TSTRIDE];
-            float cin[TC * 8];
         } a;
         struct {  // fixed-point area / height sums of half a chunk (the coverage adjoint)
             unsigned long long fa[TC / 2 * 64];
@@ -149,8 +148,7 @@ constexpr int A_SCAP = 1024;  // spans per path
 constexpr size_t A_OFF_TILES = 0;                                            // float[A_TCAP][128]: g, G
 constexpr size_t A_OFF_CMD = A_OFF_TILES + (size_t)A_TCAP * 128 * 4;         // float[A_VCAP][12]
 constexpr size_t A_OFF_CMDOFF = A_OFF_CMD + (size_t)A_VCAP * 12 * 4;         // uint32[A_VCAP + 1]
-constexpr size_t A_OFF_DW = A_OFF_CMDOFF + (size_t)(A_VCAP + 4) * 4;         // float2[A_PCAP]
-constexpr size_t A_OFF_PCMD = A_OFF_DW + (size_t)A_PCAP * 8;                 // uint32[A_PCAP]
+constexpr size_t A_OFF_PCMD = A_OFF_CMDOFF + (size_t)(A_VCAP + 4) * 4;       // uint32[A_PCAP]
 constexpr size_t A_OFF_SPANS = A_OFF_PCMD + (size_t)A_PCAP * 4;              // uint32[A_SCAP][2]
 constexpr size_t A_OFF_L64 = (A_OFF_SPANS + (size_t)A_SCAP * 8 + 255) & ~(size_t)255;  // double2[F_LCAP][2]
 constexpr size_t A_SCRATCH = A_OFF_L64 + (size_t)F_LCAP * 32;

@@ -1132,7 +1132,7 @@ static int finish_draws(ochre_rasterizer* const* rs, size_t m, const ochre_tile_
     int64_t tcap = std::max<int64_t>((int64_t)(dp->tile_alpha.bytes / 64), 64 * (int64_t)m);
     int64_t scap = std::max<int64_t>((int64_t)(dp->span_w.bytes / 2), 8 * (int64_t)m);
     const bool dense = ctx->c.dense;
-    ctx->c.dense = false;  // the ordered kernels: bit-exact, as a single finish is
+    ctx->c.dense = false;  // the plain pipeline: bit-exact, as a single finish is
     for (int attempt = 0; attempt < 2; attempt++) {
         hipError_t e;
         if ((e = dp->tile_xy.ensure(tcap * 4)) != hipSuccess || (e = dp->tile_alpha.ensure(tcap * 64)) != hipSuccess ||
