@@ -472,6 +472,7 @@ __global__ void k_scatter_ranges(const uint32_t* ids, uint32_t n, const int64_t*
 
 struct BatchedState {
     DBuf scratch, ascratch, ctl, deferred, dense_ids, dense_ids2, dense_ids3, d_sizes, d_pack;
+    DBuf adj_bin, adj_ids;       // the adjoint's path order
     DBuf large_cmd, large_grid;  // the large-path adjoint's scratch
     DBuf g_verbs, g_points, g_weights, g_xf, g_ts, g_tc, g_ss, g_sc;
     // graph of (reset, dense kernels) for the last argument set
@@ -942,6 +943,14 @@ int run_adjoint(Context* ctx, const SegInput& in, const AdjTarget& tgt, float* l
     FusedCtl* ctl = B->ctl.as<FusedCtl>();
     const uint32_t g = (uint32_t)std::max(1, gran);
     hipLaunchKernelGGL(k_fused_reset, dim3(1), dim3(64), 0, s, ctl);
+    if (NP > n_waves) {  // (up to a path per wave all start at once)
+        HIPCHK_RET(B->adj_bin.ensure((size_t)NP));
+        HIPCHK_RET(B->adj_ids.ensure((size_t)NP * 4));
+        hipLaunchKernelGGL(k_adj_weigh, dim3((uint32_t)((NP + 3) / 4)), dim3(256), 0, s, fi, B->adj_bin.as<uint8_t>());
+        hipLaunchKernelGGL(k_adj_order, dim3(1), dim3(1024), 0, s, B->adj_bin.as<uint8_t>(), NP,
+                           B->adj_ids.as<uint32_t>());
+        fi.ids = B->adj_ids.as<uint32_t>();
+    }
     if (ctx->timing) {
         if (!ctx->ev[0]) HIPCHK_RET(hipEventCreate(&ctx->ev[0]));
         if (!ctx->ev[1]) HIPCHK_RET(hipEventCreate(&ctx->ev[1]));
