@@ -2018,7 +2018,7 @@ static int run_plain_pass(Context* ctx, const SegInput& in, OutputDesc& out, hip
     HIPCHK(ctx->vals[1].ensure(std::max<int64_t>(R, 1) * 4));
     HIPCHK(ctx->records.ensure(std::max<int64_t>(RUNS, 1) * sizeof(RunRec)));
     const int rs_bits = rs_digit_bits((int)kbits);
-    const int64_t rs_tile = (int64_t)RS_NT * rs_items(R);
+    const int64_t rs_tile = (int64_t)rs_threads(rs_bits, rs_items(R)) * rs_items(R);
     const uint32_t rs_blocks = (uint32_t)std::max<int64_t>(1, (R + rs_tile - 1) / rs_tile);
     if (!unordered) HIPCHK(ctx->rs_counts.ensure(((size_t)rs_blocks << rs_bits) * 4));
     HIPCHK(ensure_scan_capacity(ctx, std::max<int64_t>({unordered ? 1 : (int64_t)rs_blocks << rs_bits, ROWS, 1})));
@@ -2147,12 +2147,12 @@ static int run_plain_pass(Context* ctx, const SegInput& in, OutputDesc& out, hip
     auto sort_pass = [&](auto bits, auto items, int shift) -> hipError_t {
         constexpr int B = decltype(bits)::value, I = decltype(items)::value;
         uint32_t *kin = ctx->keys[cur].as<uint32_t>(), *vin = ctx->vals[cur].as<uint32_t>();
-        hipLaunchKernelGGL((k_rs_count<B, I>), dim3(rs_blocks), dim3(RS_NT), 0, s, kin, R, shift, rsc, rs_blocks);
+        hipLaunchKernelGGL((k_rs_count<B, I>), dim3(rs_blocks), dim3(rs_threads(B, I)), 0, s, kin, R, shift, rsc, rs_blocks);
         const hipError_t e = launch_scan<uint32_t>(ctx, (int64_t)rs_blocks << B, LoadU32{rsc}, StoreU32{rsc}, OpAdd(),
                                                    0u, (uint32_t*)nullptr, s);
         if (e != hipSuccess) return e;
         // values are the entry payloads (a run, or crossing sign with bit 31)
-        hipLaunchKernelGGL((k_rs_scatter<B, I>), dim3(rs_blocks), dim3(RS_NT), 0, s, kin, vin, R, shift, rsc,
+        hipLaunchKernelGGL((k_rs_scatter<B, I>), dim3(rs_blocks), dim3(rs_threads(B, I)), 0, s, kin, vin, R, shift, rsc,
                            rs_blocks, ctx->keys[cur ^ 1].as<uint32_t>(), ctx->vals[cur ^ 1].as<uint32_t>());
         cur ^= 1;
         return hipSuccess;

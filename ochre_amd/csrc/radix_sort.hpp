@@ -9,8 +9,10 @@
 
 namespace ochre {
 
-constexpr int RS_NT = 256;  // threads per block
-constexpr int RS_WAVES = RS_NT / WAVE;
+// Threads per block: 512 for large inputs with 10-bit digits, where a block's 1,024
+// counts are stored and read a line apart (plain call of 10,000 glyphs: k_rs_count
+// 31.7 -> 25.1 us a pass, the call 832 -> 806).
+inline constexpr int rs_threads(int bits, int items) { return bits == 10 && items == 16 ? 512 : 256; }
 // Keys per thread: 16, or 4 for small inputs, whose blocks would otherwise be too
 // few to reach every CU (a plain call of 61 glyphs, 15,000 keys: 270 us with 4,
 // 278 with 16; 150,000 keys 308 / 326, 300,000 348 / 348, 600,000 450 / 416).
@@ -29,9 +31,9 @@ __device__ inline uint64_t lanemask_lt() {
 
 // counts[digit * nblocks + block]
 template <int BITS, int ITEMS>
-__global__ __launch_bounds__(RS_NT) void k_rs_count(const uint32_t* __restrict__ keys, int64_t n, int shift,
+__global__ __launch_bounds__(rs_threads(BITS, ITEMS)) void k_rs_count(const uint32_t* __restrict__ keys, int64_t n, int shift,
                                                     uint32_t* __restrict__ counts, uint32_t nblocks) {
-    constexpr int DIGITS = 1 << BITS;
+    constexpr int DIGITS = 1 << BITS, RS_NT = rs_threads(BITS, ITEMS), RS_WAVES = RS_NT / WAVE;
     __shared__ uint32_t hist[RS_WAVES][DIGITS];
     const int tid = threadIdx.x;
     const int wid = tid / WAVE;
@@ -62,7 +64,8 @@ __global__ __launch_bounds__(RS_NT) void k_rs_count(const uint32_t* __restrict__
 // store consecutive addresses of one digit's run.
 template <int BITS, int ITEMS>
 struct RsScatterLds {
-    static constexpr int DIGITS = 1 << BITS, TILE_KEYS = RS_NT * ITEMS;
+    static constexpr int DIGITS = 1 << BITS, RS_NT = rs_threads(BITS, ITEMS), RS_WAVES = RS_NT / WAVE,
+                         TILE_KEYS = RS_NT * ITEMS;
     uint16_t cnt[RS_WAVES][DIGITS];  // per wave and digit: count, then the wave's start within the digit
     uint16_t dstart[DIGITS];         // the digit's first position in the block
     uint32_t goff[DIGITS];           // the digit's global start for this block
@@ -72,13 +75,13 @@ struct RsScatterLds {
 };
 
 template <int BITS, int ITEMS>
-__global__ __launch_bounds__(RS_NT, 4) void k_rs_scatter(const uint32_t* __restrict__ keys_in,
+__global__ __launch_bounds__(rs_threads(BITS, ITEMS), 4) void k_rs_scatter(const uint32_t* __restrict__ keys_in,
                                                       const uint32_t* __restrict__ vals_in, int64_t n, int shift,
                                                       const uint32_t* __restrict__ offsets, uint32_t nblocks,
                                                       uint32_t* __restrict__ keys_out,
                                                       uint32_t* __restrict__ vals_out) {
     using Lds = RsScatterLds<BITS, ITEMS>;
-    constexpr int DIGITS = Lds::DIGITS, PER = DIGITS / RS_NT;  // consecutive digits per thread
+    constexpr int DIGITS = Lds::DIGITS, RS_NT = Lds::RS_NT, RS_WAVES = Lds::RS_WAVES, PER = DIGITS / RS_NT;  // consecutive digits per thread
     __shared__ Lds s;
     const int tid = threadIdx.x;
     const int wid = tid / WAVE;
