@@ -1496,13 +1496,12 @@ static_assert(RT_ROWS * RT_NW == TILE && RT_ROWS <= 2, "the carry takes one or t
 constexpr int RT_U = 2;  // entries per thread whose loads are issued together
 
 // The window's per-pixel sums are fixed point (fx_of: 64-bit integers in units of
-// 2^-30): the sums of the increments (|area|, |height| <= 1 +
-// a few ulps, each truncated at 2^-30) are then exact, so that the decoded f32
-// sum is the correctly rounded sum of the increments, independent of arrival
-// order.  A window of a full-range path (coordinates that may be huge or
-// non-finite) or with 2^22 entries or more keeps f32 atomics in the slots' low
-// words instead.
-constexpr uint32_t RT_FX_MAX_ENTRIES = 1u << 22;  // a pixel takes at most one increment per run: < 2^22 x (1 + ulps) < 2^23
+// 2^-30): the sums of the increments, each truncated at 2^-30, are then exact, so
+// that the decoded f32 sum is the correctly rounded sum of the increments,
+// independent of arrival order.  A window of a full-range path (coordinates that may
+// be huge or non-finite) or with 2^22 entries or more keeps f32 atomics in the slots'
+// low words instead.
+constexpr uint32_t RT_FX_MAX_ENTRIES = 1u << 22;  // (a pixel takes at most one increment per run)
 
 template <bool EMIT>
 struct RowLds {
@@ -1515,9 +1514,28 @@ struct RowLds {
     uint32_t nt, ns, nocc;
 };
 
+// The increments of a run into a window's fixed-point sums (xb: the first slot of
+// its tile).  Such a window's path is within +-HUGE_COORD, so FastWalk covers its
+// lines.
+template <bool WIDE, bool EMIT>
+__device__ inline void rt_replay_fx(RowLds<EMIT>& s, const Dda& d, V2 p0, uint32_t xb, uint32_t at, uint32_t xd,
+                                    uint32_t yd) {
+    FastWalk w;
+    w.init(d, p0);
+    for (;;) {  // (at most 15 steps: each moves one pixel on, the same way along its axis)
+        float area, height;
+        bool y;
+        const bool end = w.step(area, height, y);
+        const uint32_t px = xb + at - ((at >> 4) << 3);
+        atomicAdd(reinterpret_cast<unsigned long long*>(&s.acc_a[px]), fx_of<WIDE>(area));
+        atomicAdd(reinterpret_cast<unsigned long long*>(&s.acc_h[px]), fx_of<WIDE>(height));
+        at += y ? yd : xd;
+        if (end || (at & 0x88u)) break;
+    }
+}
+
 // Replays a run (x: its tile within the window) into the window's LDS sums, in
-// arrival order: fixed point where fx, else float atomics.  In an fx window every
-// path is within +-HUGE_COORD, so FastWalk covers its lines.
+// arrival order.
 template <bool EMIT>
 __device__ inline void rt_replay_run(RowLds<EMIT>& s, uint32_t x, const RunRec& rr, const float4& L, bool fx,
                                      Counters* cnt) {
@@ -1540,19 +1558,9 @@ __device__ inline void rt_replay_run(RowLds<EMIT>& s, uint32_t x, const RunRec& 
     uint32_t at = (uint32_t)(((d.y & 7) << 4) | (d.x & 7));
     const uint32_t xd = (uint32_t)(int32_t)d.x_dir, yd = (uint32_t)((int32_t)d.y_dir * 16);
     const uint32_t xb = x * (uint32_t)UWS;
-    if (fx) {
-        FastWalk w;
-        w.init(d, p0);
-        for (;;) {  // (at most 15 steps: each moves one pixel on, the same way along its axis)
-            float area, height;
-            bool y;
-            const bool end = w.step(area, height, y);
-            const uint32_t px = xb + at - ((at >> 4) << 3);
-            atomicAdd(reinterpret_cast<unsigned long long*>(&s.acc_a[px]), fx_of(area));
-            atomicAdd(reinterpret_cast<unsigned long long*>(&s.acc_h[px]), fx_of(height));
-            at += y ? yd : xd;
-            if (end || (at & 0x88u)) break;
-        }
+    if (fx) {  // (a step along an axis is 1 / the line's length there)
+        if (__ballot(fminf(d.x_step, d.y_step) < 1.0f / FX_NARROW_PX) == 0) rt_replay_fx<false>(s, d, p0, xb, at, xd, yd);
+        else rt_replay_fx<true>(s, d, p0, xb, at, xd, yd);
         return;
     }
     const bool finite = line_finite(last, point);

@@ -169,16 +169,28 @@ struct BoxAcc {
 };
 
 // Per-pixel sums of the unordered tile stage in fixed point, 64-bit integers in
-// units of 2^-30: an increment's |area|, |height| <= 1 plus the rounding of
-// coordinates within +-30000 (below 2), so it converts through 32 bits (a
-// multiplication, a truncation and the sign: half the cost of the same in f64), and
-// the sums of 2^22 of them stay below 2^53 units; the sum is then independent of
-// arrival order, and the decoded f32 value is the correctly rounded sum of the
-// increments (each truncated at 2^-30).
+// units of 2^-30: each increment is truncated there, and the sum is then independent
+// of arrival order; below 2^53 units the decoded f32 value is the correctly rounded
+// sum.
+//
+// An increment's |height| is at most a pixel's plus rounding, but its |area| is not:
+// a crossing parameter is a sum of up to span steps (the line's longer axis in
+// pixels), each rounded by up to 2^-25, so the walk's pixel and the line's point
+// drift apart by up to d = span^2 * 2^-25 px (plus 0.01 px of rounding of coordinates
+// within +-30000), and |area| <= (1 + 0.02) * (1 + d).  Lines of up to FX_NARROW_PX
+// (d = 0.5, |area| < 1.6) convert through 32 bits, a multiplication, a truncation and
+// the sign, half the cost of the same in f64; longer ones (d up to 107 px at 60,000,
+// |area| up to 11 measured at 30,000) through 64.  Sums of 2^22 increments of at most
+// 2^7 fit 64 bits.
+constexpr float FX_NARROW_PX = 4096.0f;
 constexpr float FX_SCALE = 1073741824.0f;           // 2^30
 constexpr double FX_UNIT = 9.313225746154785e-10;  // 2^-30
 
-__device__ inline unsigned long long fx_of(float v) { return (unsigned long long)(long long)(int32_t)(v * FX_SCALE); }
+template <bool WIDE>
+__device__ inline unsigned long long fx_of(float v) {
+    if constexpr (WIDE) return (unsigned long long)(long long)(v * FX_SCALE);
+    return (unsigned long long)(long long)(int32_t)(v * FX_SCALE);
+}
 __device__ inline float fx_to_f(long long q) { return (float)((double)q * FX_UNIT); }
 
 // ------------------------------------------------------ (b) DDA binning
