@@ -492,11 +492,13 @@ struct BatchedState {
 // gets the context's own limits.
 static int run_plain_bounded(Context* ctx, const SegInput& in, OutputDesc& out, hipStream_t s) {
     const OutputDesc asked = out;
-    int st = run_plain(ctx, in, out, s, false, (int64_t)1 << 23, (int64_t)1 << 24);
+    SegInput si = in;
+    si.own_ranges = true;
+    int st = run_plain(ctx, si, out, s, false, (int64_t)1 << 23, (int64_t)1 << 24);
     if (st == -2) {
         (void)hipGetLastError();
         out = asked;
-        st = run_plain(ctx, in, out, s, false, (int64_t)1 << 20, (int64_t)1 << 21);
+        st = run_plain(ctx, si, out, s, false, (int64_t)1 << 20, (int64_t)1 << 21);
     }
     return st;
 }
@@ -737,6 +739,7 @@ int run_batched(Context* ctx, const SegInput& in, OutputDesc& out, hipStream_t s
         si.n_verbs = dv[nd];
         si.n_points = dp[nd];
         si.n_weights = dw[nd];
+        si.own_ranges = true;
         OutputDesc od;
         const bool room = Tf <= out.tile_capacity && Sf <= out.span_capacity;
         od.tile_xy = out.tile_xy + (room ? 2 * Tf : 0);

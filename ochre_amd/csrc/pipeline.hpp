@@ -31,6 +31,12 @@ struct SegInput {
     const int32_t* seg_path = nullptr;       // [n_segs] or null (segment i -> path i)
     const int64_t* path_seg_off = nullptr;   // [n_paths + 1] or null (identity)
     int64_t n_verbs = 0, n_points = 0, n_weights = 0;
+    // The batched call's paths (segment i is path i): each is its own range of the
+    // input, wherever its offsets put that; its verbs consume exactly its points,
+    // and weights that they leave are ignored.  Without this the ranges follow one
+    // another from the arrays' start, and a range's surplus is found at the next
+    // one's first verb.
+    bool own_ranges = false;
 };
 
 struct OutputDesc {

@@ -188,16 +188,30 @@ __device__ inline Cmd resolve_cmd(const SegInput& in, const CmdAcc* scan, int64_
     int64_t vb = in.seg_verb_off[fs], ve = in.seg_verb_off[ls];
     int64_t pb = in.seg_point_off[fs];
     CmdAcc a = scan[i];
-    int64_t g = a.pts;
+    // the point and weight cursors, and the ends of what they may reach; the
+    // scanned ones count from the arrays' start, a path's own from its first verb
+    CmdAcc base{0, 0, -1, 0};
+    int64_t p0 = 0, w0 = 0, p_end = in.n_points, w_end = in.n_weights;
+    if (in.own_ranges) {
+        base = scan[vb];
+        p0 = pb;
+        p_end = in.seg_point_off[s + 1];
+        w0 = in.seg_weight_off[s];
+        w_end = in.seg_weight_off[s + 1];
+    }
+    const int64_t g = p0 + (a.pts - base.pts);
     c.path = (int32_t)p;
     c.verb = in.verbs[i];
     c.last_in_path = (i == ve - 1);
     int np = verb_points(c.verb);
     c.bad = np < 0;
-    if (i == in.seg_verb_off[s] && (g != in.seg_point_off[s] || (int64_t)a.conics != in.seg_weight_off[s]))
-        c.bad = true;
     if (np < 0) np = 0;
-    if (g + np > in.n_points) {
+    if (in.own_ranges) {
+        if (c.last_in_path && g + np != p_end) c.bad = true;
+    } else if (i == in.seg_verb_off[s] && (g != in.seg_point_off[s] || (int64_t)a.conics != in.seg_weight_off[s])) {
+        c.bad = true;
+    }
+    if (g + np > p_end) {
         c.bad = true;
         np = 0;
     }
@@ -207,10 +221,13 @@ __device__ inline Cmd resolve_cmd(const SegInput& in, const CmdAcc* scan, int64_
     if (np > 2) c.pt[2] = load_point(in, g + 2, s);
     c.w = 0.0f;
     if (c.verb == CONIC) {
-        if ((int64_t)a.conics < in.n_weights) c.w = in.weights[a.conics];
+        const int64_t wi = w0 + (a.conics - base.conics);
+        if (wi < w_end) c.w = in.weights[wi];
         else c.bad = true;
     }
-    if (g > pb) {
+    if (g > p_end) {  // (bad already)
+        c.start = mk(0.0f, 0.0f);
+    } else if (g > pb) {
         int64_t sp = (g - 1 >= in.seg_point_off[s]) ? s : seg_search(in.seg_point_off, in.n_segs, g - 1);
         c.start = load_point(in, g - 1, sp);
     } else {
@@ -218,13 +235,28 @@ __device__ inline Cmd resolve_cmd(const SegInput& in, const CmdAcc* scan, int64_
     }
     if (a.move >= vb) {
         int64_t ms = a.move >= in.seg_verb_off[s] ? s : seg_search(in.seg_verb_off, in.n_segs, a.move);
-        int64_t gm = scan[a.move].pts;
-        if (gm < in.n_points) c.first = load_point(in, gm, ms);
+        const int64_t gm = p0 + (scan[a.move].pts - base.pts);
+        if (gm < p_end) c.first = load_point(in, gm, ms);
         else c.bad = true;
     } else {
         c.first = mk(0.0f, 0.0f);
     }
     return c;
+}
+
+// Whether command i belongs to a path (own ranges may leave some before and after).
+__device__ inline bool in_paths(const SegInput& in, int64_t i) {
+    return i < in.n_verbs &&
+           (!in.own_ranges || (i >= in.seg_verb_off[0] && i < in.seg_verb_off[in.n_segs]));
+}
+
+// The paths' boxes, empty.  A path of its own range without verbs has no points either.
+__global__ void k_path_init(SegInput in, PathBox* box, Counters* cnt) {
+    const int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (p >= in.n_paths) return;
+    box[p] = PathBox{INT32_MAX, INT32_MAX, INT32_MIN, INT32_MIN, 0, {0, 0, 0}};
+    if (in.own_ranges && in.seg_verb_off[p] == in.seg_verb_off[p + 1] && in.seg_point_off[p] != in.seg_point_off[p + 1])
+        atomicOr(&cnt->error, (uint32_t)ERR_INPUT);
 }
 
 struct FlattenArgs {
@@ -276,10 +308,13 @@ __global__ __launch_bounds__(256) void k_flatten(FlattenArgs a) {
         const int64_t i0 = (int64_t)blockIdx.x * FL_CMDS;
         const int nb = (int)min<int64_t>((int64_t)FL_CMDS, a.in.n_verbs - i0);
         if (in_range) {
+            foff[t] = a.cmd_line_off[i];
+            if (t == nb - 1) foff[nb] = foff[t] + a.cmd_lines[i];
+            fc[t].info = 0xfu;  // no lines
+        }
+        if (in_range && in_paths(a.in, i)) {
             const Cmd c = resolve_cmd(a.in, a.scan, i, a.cmd_seg[i]);
-            const uint32_t o = a.cmd_line_off[i];
-            foff[t] = o;
-            if (t == nb - 1) foff[nb] = o + a.cmd_lines[i];
+            const uint32_t o = foff[t];
             FlatCmd f;
             f.start = make_float2(c.start.x, c.start.y);
             f.p0 = make_float2(c.pt[0].x, c.pt[0].y);
@@ -387,7 +422,9 @@ __global__ __launch_bounds__(256) void k_flatten(FlattenArgs a) {
     int32_t key = -1;
     uint32_t n = 0, flags = 0;
     BoxAcc box;
-    if (in_range) {
+    if (in_range && !in_paths(a.in, i)) {
+        a.cmd_lines[i] = 0;
+    } else if (in_range) {
         const int64_t sg = seg_search_wave(a.in.seg_verb_off, a.in.n_segs, i);
         a.cmd_seg[i] = (uint32_t)sg;
         Cmd c = resolve_cmd(a.in, a.scan, i, sg);
@@ -1925,14 +1962,7 @@ static int run_plain_pass(Context* ctx, const SegInput& in, OutputDesc& out, hip
     HIPCHK(ctx->path_rows.ensure(NP * 4));
     CmdAcc* cscan = ctx->cmd_scan.as<CmdAcc>();
     PathBox* box = ctx->path_box.as<PathBox>();
-    {
-        PathBox init;
-        init.minx = init.miny = INT32_MAX;
-        init.maxx = init.maxy = INT32_MIN;
-        init.flags = 0;
-        init.pad[0] = init.pad[1] = init.pad[2] = 0;
-        fill<PathBox>(box, NP, init, s);
-    }
+    hipLaunchKernelGGL(k_path_init, dim3(grid_for(NP, 256)), dim3(256), 0, s, in, box, cnt);
     HIPCHK(launch_scan<CmdAcc>(ctx, V, LoadCmd{in.verbs}, StoreCmd{cscan}, OpCmd(), CmdAcc{0, 0, -1, 0},
                                (CmdAcc*)nullptr, s));
     FlattenArgs fa;
@@ -2373,6 +2403,7 @@ int run_plain(Context* ctx, const SegInput& in, OutputDesc& out, hipStream_t s, 
         si.n_verbs = voff[p1] - voff[p0];
         si.n_points = poff[p1] - poff[p0];
         si.n_weights = woff[p1] - woff[p0];
+        si.own_ranges = in.own_ranges;
         OutputDesc od;
         od.tile_xy = out.tile_xy + (room ? 2 * T : 0);
         od.tile_alpha = out.tile_alpha + (room ? 64 * T : 0);
