@@ -42,6 +42,7 @@ struct FusedIn {
     // k_dense) instead of 0 .. n_paths
     const uint32_t* ids = nullptr;
     const uint32_t* n_ids = nullptr;
+    int64_t item_cap = F_LCAP;  // lines per chunk of commands over which a dense instance hands a path on
 };
 
 struct FusedOut {
@@ -566,6 +567,9 @@ int run_batched(Context* ctx, const SegInput& in, OutputDesc& out, hipStream_t s
     // launch: a path's latency is all there is (61 glyphs of 12-48 px 81 -> 68 us a
     // call, 256 of them 91 -> 71, 61 of 60-120 px 264 -> 238; at 512 paths, two to a
     // CU one after the other, 95 -> 108).
+    // Its chunks are of 1,024 commands, four of the 64-tile instance's, and hold four
+    // times the lines (200 paths of 1,000 cubics and 20,000 lines in 36 tiles: 279 us
+    // a call, handed on for their 8,192 lines a chunk 602; one of them 262 / 346).
     if (n_large && NP <= cus) {
         stages[n_stages++] = D_FEW;
     } else {
@@ -580,6 +584,7 @@ int run_batched(Context* ctx, const SegInput& in, OutputDesc& out, hipStream_t s
     uint32_t* counts[3] = {&ctl->dq, &ctl->dq2, &ctl->dq3};
     uint32_t* queues[3] = {&ctl->queue, &ctl->queue3, &ctl->queue4};
     FusedIn fin[3] = {fi, fi, fi};  // stage i reads fin[i]
+    if (stages[0] == D_FEW) fin[0].item_cap = 4 * (int64_t)F_LCAP;
     for (int i = 1; i < n_stages; i++) {
         fin[i].ids = lists[i - 1];
         fin[i].n_ids = counts[i - 1];
