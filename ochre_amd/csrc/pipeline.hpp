@@ -119,6 +119,9 @@ struct AtlasState {
 // a segment input (several fills per path), returns -7.
 constexpr int64_t PLAIN_MAX_LINES = 1ll << 29;
 constexpr int64_t PLAIN_MAX_ENTRIES = 1ll << 30;
+// What a path of the batched call may have whatever the context's limits are: the
+// lines of a path within 32 x 32 tiles, each at most 63 runs and 32 crossings.
+constexpr int64_t OWN_MIN_LINES = 8192, OWN_MIN_ENTRIES = OWN_MIN_LINES * 95;
 
 struct Context {
     int device = 0;

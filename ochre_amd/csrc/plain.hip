@@ -2336,16 +2336,17 @@ int run_plain(Context* ctx, const SegInput& in, OutputDesc& out, hipStream_t s, 
     HIPCHK(ctx->call_error.ensure(256));
     if (!ctx->host_pinned) HIPCHK(hipHostMalloc(&ctx->host_pinned, 4096));
     fill<uint32_t>(ctx->call_error.as<uint32_t>(), 1, 0u, s);
-    // a pass within the asked limits; one path over them, within the context's
+    // a pass within the asked limits; one path over them, within the context's (and,
+    // in the batched call, at least OWN_MIN_LINES and OWN_MIN_ENTRIES)
     auto pass = [&](const SegInput& si, OutputDesc& od) {
         ctx->pass_lines = pass_lines ? std::min(pass_lines, ctx->max_lines) : ctx->max_lines;
         ctx->pass_entries = pass_entries ? std::min(pass_entries, ctx->max_entries) : ctx->max_entries;
         const int rc = run_plain_pass(ctx, si, od, s, unordered);
-        if (rc != ST_SPLIT || si.n_paths > 1 ||
-            (ctx->pass_lines == ctx->max_lines && ctx->pass_entries == ctx->max_entries))
-            return rc;
-        ctx->pass_lines = ctx->max_lines;
-        ctx->pass_entries = ctx->max_entries;
+        const int64_t lines = si.own_ranges ? std::max(ctx->max_lines, OWN_MIN_LINES) : ctx->max_lines;
+        const int64_t entries = si.own_ranges ? std::max(ctx->max_entries, OWN_MIN_ENTRIES) : ctx->max_entries;
+        if (rc != ST_SPLIT || si.n_paths > 1 || (ctx->pass_lines >= lines && ctx->pass_entries >= entries)) return rc;
+        ctx->pass_lines = lines;
+        ctx->pass_entries = entries;
         return run_plain_pass(ctx, si, od, s, unordered);
     };
     int st = pass(in, out);

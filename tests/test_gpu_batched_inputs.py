@@ -133,7 +133,22 @@ def test_missing_points_are_refused(gpu_ctx, where, short, mode):
     assert _status(gpu_ctx, b, mode) == -1
 
 
-@pytest.mark.parametrize("limits", [(0, 0), (1000, 0), (0, 8000)])
+@pytest.mark.parametrize("mode", MODES)
+@pytest.mark.parametrize("limits", [(16, 64), (0, 64), (16, 0)])
+def test_small_pass_limits_refuse_no_small_path(gpu_ctx, limits, mode):
+    """The plain pipeline's pass limits cut a batch into ranges; a path of up to 8,192 lines
+    within 32 x 32 tiles is rasterised by the batched call whatever they are."""
+    from ochre_amd.device import run_to_host, set_pass_limits
+    b = W.concat([W.glyph_run(4, seed=51), _large(52), W.from_paths([_conics(53)], W.IDENTITY), _large(54)])
+    set_pass_limits(gpu_ctx, *limits)
+    try:
+        got = run_to_host(gpu_ctx, b, mode, 4096, 4096)
+    finally:
+        set_pass_limits(gpu_ctx, 0, 0)
+    compare(oracle_ref.run_batch(b), got, max_lsb=1 if mode == "dense" else 0)
+
+
+@pytest.mark.parametrize("limits", [(0, 0), (1000, 0), (0, 8000), (60, 500)])
 @pytest.mark.parametrize("n", [1, 3, 40])
 def test_ordered_batches_against_the_oracle(gpu_ctx, n, limits):
     """The call with the dense kernels off, in one pass and in several, and with outputs that
