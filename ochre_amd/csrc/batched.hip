@@ -516,6 +516,15 @@ __global__ void k_defer_sizes(FusedIn in, const uint32_t* ids, uint32_t n, Defer
                        in.weight_off[p + 1] - in.weight_off[p]};
 }
 
+static bool few_paths(const Context* ctx, int64_t n_paths, int cus) { return ctx->dense_large && n_paths <= cus; }
+
+bool few_paths_route(const Context* ctx, int64_t n_paths) {
+    int cus = 0;
+    return ctx->dense && n_paths > 0 &&
+           hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device) == hipSuccess &&
+           few_paths(ctx, n_paths, cus);
+}
+
 int run_batched(Context* ctx, const SegInput& in, OutputDesc& out, hipStream_t s, bool use_graph) {
     if (!ctx->batched) ctx->batched = new BatchedState();
     BatchedState* B = reinterpret_cast<BatchedState*>(ctx->batched);
@@ -570,7 +579,7 @@ int run_batched(Context* ctx, const SegInput& in, OutputDesc& out, hipStream_t s
     // Its chunks are of 1,024 commands, four of the 64-tile instance's, and hold four
     // times the lines (200 paths of 1,000 cubics and 20,000 lines in 36 tiles: 279 us
     // a call, handed on for their 8,192 lines a chunk 602; one of them 262 / 346).
-    if (n_large && NP <= cus) {
+    if (few_paths(ctx, NP, cus)) {
         stages[n_stages++] = D_FEW;
     } else {
         if (n_small) stages[n_stages++] = D_SMALL;

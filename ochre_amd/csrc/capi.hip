@@ -394,7 +394,15 @@ int ochre_autotune_batched(ochre_context* ctx, const ochre_path_batch* in, ochre
         *ms_out = (float)t[t.size() / 2];
         return 0;
     };
-    if (ctx->c.dense) {
+    if (few_paths_route(&ctx->c, in->n_paths)) {  // one launch shape, which no setting changes
+        float ms = 0;
+        st = measure(&ms);
+        if (st) return st;
+        if (results && k < max_results)
+            results[k] = ochre_batched_tuning{best.waves_per_cu, best.paths_per_pop, best.tiles_per_chunk, ms, best_dg,
+                                              best_dw, ctx->c.dense_small_groups, ctx->c.dense_large};
+        k++;
+    } else if (ctx->c.dense) {
         for (int dg : dgroups)
             for (int dw : dwaves) {
                 if (dw == 8 && dg > 2) continue;  // 16 waves of 128 registers fill a CU
@@ -495,9 +503,10 @@ std::string tune_key(const Context& c, const ochre_path_batch* in) {
         if (ch == ' ' || ch == '=') ch = '_';
     const double np = (double)std::max<int64_t>(in->n_paths, 1);
     char buf[256];
-    snprintf(buf, sizeof buf, "%s/cu%d/dense%d/paths%d/verbs%d/points%d", name.c_str(), cus, c.dense ? 1 : 0,
+    // (a batch that the few-paths instance takes apart from others of its bucket)
+    snprintf(buf, sizeof buf, "%s/cu%d/dense%d/paths%d/verbs%d/points%d%s", name.c_str(), cus, c.dense ? 1 : 0,
              bucket((double)in->n_paths, 1.0), bucket((double)in->n_verbs / np, 2.0),
-             bucket((double)in->n_points / np, 2.0));
+             bucket((double)in->n_points / np, 2.0), few_paths_route(&c, in->n_paths) ? "/few" : "");
     return buf;
 }
 
@@ -541,7 +550,7 @@ int ochre_autotune_batched_cached(ochre_context* ctx, const ochre_path_batch* in
             ctx->c.batched_gran = e.gran;
             ctx->c.batched_tc = e.tc;
             ctx->c.batched_graph = true;
-            if (ctx->c.dense) {
+            if (ctx->c.dense && !few_paths_route(&ctx->c, in->n_paths)) {  // (few paths: other batches' settings stay)
                 ctx->c.dense_groups_per_cu = e.dense_groups;
                 ctx->c.dense_waves = e.dense_waves;
                 ctx->c.dense_small_groups = e.dense_small;

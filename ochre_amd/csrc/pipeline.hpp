@@ -179,6 +179,9 @@ int run_plain(Context* ctx, const SegInput& in, OutputDesc& out, hipStream_t str
 // use_graph replays the dense launches from a captured HIP graph where a call
 // repeats the one before.
 int run_batched(Context* ctx, const SegInput& in, OutputDesc& out, hipStream_t stream, bool use_graph);
+// Whether run_batched takes a batch of so many paths by the 16-wave dense instance
+// alone, whose launch no setting but dense and dense_large changes.
+bool few_paths_route(const Context* ctx, int64_t n_paths);
 // One path by k_single with no host round trip: the output goes where `out`
 // points and the control block (SMALL_CTL_BYTES, reset by the kernel) to
 // `ctl`, both device-visible (pinned host memory mapped into the device's
