@@ -64,8 +64,8 @@ def test_tuning_key_tells_the_two_routes_apart(gpu_ctx, tmp_path):
     """As many paths as compute units and a few more lie in one power of two; only the
     second batch uses the tuned shapes."""
     import torch
-    from ochre_amd.device import (Context, DeviceOutput, autotune_cached, dense_params, set_dense_params, set_dense_small,
-                                  upload)
+    from ochre_amd.device import (Context, DeviceOutput, autotune_cached, dense_params, set_dense_large, set_dense_params,
+                                  set_dense_small, upload)
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     if (cus + 1).bit_length() != cus.bit_length():
         pytest.skip("one more path is another power of two")
@@ -80,6 +80,7 @@ def test_tuning_key_tells_the_two_routes_apart(gpu_ctx, tmp_path):
         tuned = dense_params(ctx)
         assert len(open(path).read().splitlines()) == 2
         # found again: the first one leaves what the context has, the second sets the shapes
+        set_dense_large(ctx, True)  # (tuning the second may have chosen otherwise)
         set_dense_params(ctx, True, 3, 2)
         set_dense_small(ctx, 6)
         mine = dense_params(ctx)
