@@ -119,7 +119,13 @@ void ochre_rasterizer_free(ochre_rasterizer* r);
 
 /* Device-resident input: n_paths paths, each filled with its own transform.
  * All pointers are device pointers; *_off arrays have n_paths + 1 entries
- * (offsets in elements: verbs, points (pairs), weights). */
+ * (offsets in elements: verbs, points (pairs), weights).  A path whose verbs
+ * consume more points or weights than it has returns OCHRE_ERR_INVALID_ARG.  In
+ * the batched calls, in strokes and in the adjoint a path is its own range by the
+ * offsets, which may start at a later path of the arrays; points left over return
+ * OCHRE_ERR_INVALID_ARG, weights left over are ignored.  ochre_rasterize_plain
+ * takes the ranges one after another from the arrays' start and compares the
+ * consumed points and weights with the offsets at each path's first verb. */
 typedef struct ochre_path_batch {
     int64_t n_paths;
     const uint8_t* verbs;
@@ -195,8 +201,8 @@ int ochre_rasterize_batched(ochre_context* ctx, const ochre_path_batch* in, ochr
  * read the counters back.  Limits: at most 2^20 paths per call
  * (OCHRE_ERR_TOO_LARGE before anything runs); a path over the 256-tile
  * instance (a tile grid of more than 256 tiles or 32 on a side, more than
- * 128 lines over 8 pixel steps, a conic weight that is not positive and
- * finite) makes the call return OCHRE_ERR_TOO_LARGE after the other paths are
+ * 8,192 lines from a chunk of 256 or 1,024 commands, a conic weight that is not
+ * positive and finite) makes the call return OCHRE_ERR_TOO_LARGE after the other paths are
  * written, with that path's range unwritten (ochre_rasterize_batched handles
  * it).  Every call on a device shares that device's array, which keeps the
  * last call's contents; each call clears the counters it uses, and calls that
@@ -247,14 +253,16 @@ int ochre_context_set_batched_params(ochre_context* ctx, int waves_per_cu, int p
 int ochre_context_get_batched_params(ochre_context* ctx, int* waves_per_cu, int* paths_per_pop, int* tiles_per_chunk,
                                      int* use_graph);
 
-/* The dense single-walk kernel (on by default) takes every path whose tile grid (line bounding box + a 2 px
- * margin) has at most 64 tiles: one DDA walk adds each increment to its
- * pixel's sums with LDS float atomics, so f32 sums are taken in arrival
+/* The dense single-walk kernel (on by default) takes every path whose tile grid
+ * (line bounding box + a 2 px margin) has at most 64 tiles: one DDA walk adds each
+ * increment to its pixel's sums with LDS float atomics, so f32 sums are taken in arrival
  * order and an alpha can differ from the ordered result by 1 LSB (tile and
  * span sets are exact).  Off: every path goes through the plain pipeline,
  * whose sums follow emission order.  groups_per_cu 1-8 resident workgroups,
  * waves_per_group 2, 4 or 8 (waves sharing one path; with 8, at most 2
- * workgroups per CU are resident). */
+ * workgroups per CU are resident).  A batch of at most one path per compute unit
+ * runs a 256-tile instance of 16 waves alone while dense_large is on: then neither
+ * these two settings nor dense_small change the call. */
 int ochre_context_set_dense_params(ochre_context* ctx, int enabled, int groups_per_cu, int waves_per_group);
 int ochre_context_get_dense_params(ochre_context* ctx, int* enabled, int* groups_per_cu, int* waves_per_group);
 /* A small-grid dense instance (tile grids of at most 32 tiles, 2 waves and
@@ -267,7 +275,8 @@ int ochre_context_get_dense_small(ochre_context* ctx, int* groups_per_cu);
 /* A 256-tile dense instance (one workgroup of 8 waves and 140 KB of LDS per
  * CU) behind the 64-tile one, over the paths it hands on (grids of 65-256
  * tiles go there instead of to the plain pipeline); enabled 0 or 1, default
- * 1.  The autotuner tries both. */
+ * 1.  The autotuner tries both.  A batch of at most one path per compute unit
+ * runs it with 16 waves and nothing in front. */
 int ochre_context_set_dense_large(ochre_context* ctx, int enabled);
 int ochre_context_get_dense_large(ochre_context* ctx, int* enabled);
 
@@ -275,7 +284,8 @@ int ochre_context_get_dense_large(ochre_context* ctx, int* enabled);
  * flattened lines and max_entries sort entries (defaults 2^29 and 2^30, about
  * 66 GB of intermediates at both).  A batch over either is rasterised as
  * consecutive path ranges into the same output, with the same result; a
- * single path over them returns OCHRE_ERR_TOO_LARGE.  0 restores a default;
+ * single path over them returns OCHRE_ERR_TOO_LARGE (in the batched calls only a
+ * path of more than 8,192 lines or 778,240 sort entries).  0 restores a default;
  * values above the defaults are clamped to them.  Tests lower the limits to
  * exercise the split on small batches.  No reference counterpart (the
  * reference holds every increment of one path in host memory). */
@@ -312,7 +322,9 @@ int ochre_coverage_adjoint(ochre_context* ctx, const ochre_path_batch* in, const
  * {1,2,3,4}, waves per workgroup {2,4,8}) of the 64-tile dense launch, then
  * the small-grid instance {off, 4, 6, 8 workgroups per CU}, the 256-tile
  * instance {off, on}; with it off the call has no launch shape, and is timed
- * once.  Each configuration is
+ * once, as is a batch of at most one path per compute unit with the 256-tile
+ * instance on, which uses none of these shapes and leaves them as they are.
+ * Each configuration is
  * timed on the caller's batch (`reps` calls, median); the fastest is kept in
  * the context and every measurement reported in `results` (up to
  * max_results entries). */

@@ -125,7 +125,7 @@ __device__ inline uint32_t tile_rank(const S& s, int tx, int ty) {
     return s.row_rank[ty] + (uint32_t)__popc(s.occ[ty] & ((1u << tx) - 1u));
 }
 
-// Adjoint inputs/outputs (see adjoint.hip).  The target of path p is its
+// Adjoint inputs/outputs (see adjoint.inc).  The target of path p is its
 // tiles [tt_start[p], +tt_count[p]) (row-major, 64 f32 coverages each) and
 // spans [ts_start[p], +ts_count[p]).
 struct AdjArgs {

@@ -1023,10 +1023,9 @@ int ochre_rasterizer_finish(ochre_rasterizer* r, const ochre_tile_builder* build
             od.path_span_start = dp->pss.as<int64_t>();
             od.path_span_count = dp->psc.as<int32_t>();
             if (one_fill) {
-                // one fill (the reference's demo makes a Rasterizer per fill):
-                // the ordered batched kernel, bit-exact like the plain pipeline,
-                // in one launch and one host synchronisation; a path over its
-                // limits goes to the plain pipeline within the call
+                // one fill (the reference's demo makes a Rasterizer per fill)
+                // over the single-fill kernel's limits: the batched call without
+                // the dense kernels, bit-exact
                 SegInput s1 = si;
                 s1.seg_path = nullptr;
                 s1.path_seg_off = nullptr;

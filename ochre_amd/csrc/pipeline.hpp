@@ -160,7 +160,7 @@ struct Context {
     int dense_groups_per_cu = 4;
     int dense_waves = 4;
     int dense_small_groups = 0;  // small-grid instance in front (0: off)
-    int dense_large = 1;         // 256-tile instance behind (1 workgroup of 8 waves per CU; 0: off)
+    int dense_large = 1;         // 256-tile instance (0: off): behind, 8 waves per CU; few paths, 16 waves alone
     StrokeBuffers stroke;
     AtlasState atlas;
     ~Context();
@@ -169,7 +169,8 @@ struct Context {
 // The plain five-kernel pipeline; see the per-pass limits above.
 // `unordered` (used for the paths the batched pipeline hands on, under the
 // dense kernels' 1-LSB contract) replaces the sort and the ordered tile pass
-// by window buckets and LDS float-atomic sums.
+// by window buckets and fixed-point LDS sums (f32 atomics in windows of
+// full-range paths or of 2^22 entries and more).
 // pass_lines / pass_entries bound a pass below the context's limits (0: no
 // further): a batch over them is split, a single path over them is not refused.
 int run_plain(Context* ctx, const SegInput& in, OutputDesc& out, hipStream_t stream, bool unordered = false,

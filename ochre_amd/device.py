@@ -312,7 +312,8 @@ def set_pass_limits(ctx: Context, max_lines=0, max_entries=0):
 
 
 def set_dense_large(ctx: Context, enabled=True):
-    """The 256-tile dense instance behind the 64-tile one."""
+    """The 256-tile dense instance: behind the 64-tile one, or alone for a batch of
+    at most one path per compute unit."""
     _lib.check(ctx.lib.ochre_context_set_dense_large(ctx.h, 1 if enabled else 0), "set_dense_large")
 
 
